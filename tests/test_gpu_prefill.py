@@ -214,6 +214,31 @@ def test_rows_gemm_row_scales(P, typ, mag):
     assert ok, max_violation(g, o)
 
 
+@pytest.mark.parametrize("typ", [GGML_Q4_0, GGML_Q8_0])
+@pytest.mark.parametrize("M,rows,cols", [
+    (1, 1, 32), (17, 300, 128), (32, 96, 544), (33, 33, 1120), (65, 4096, 96), (96, 2080, 544),
+    (129, 21984, 64), (161, 11233, 160), (500, 4064, 288), (512, 4096, 96), (1025, 8224, 32), (2048, 4097, 96)])
+def test_rows_gemm_splits(P, typ, M, rows, cols):
+    """Every split of the prompt GEMM (64 x 32 and 64 x 64 with K over 8
+    wavefronts, 64 x 128 with K over 4, 64 x 256 with K whole) at ragged rows,
+    columns and K (one block, odd block counts, fewer pairs than K slices).
+    Bound per output: two fp16 parts keep each activation to 2^-22 of its
+    row's largest, and the fp32 sums round once per 16 products and twice per
+    block (the last term: at most 2^-24 of the sum of magnitudes each)."""
+    print(f"rows gemm split {'Q4_0' if typ == GGML_Q4_0 else 'Q8_0'} {M}x{rows}x{cols}", flush=True)
+    rng = np.random.default_rng(M + rows + cols + typ)
+    W = N.rand_q4_0(rng, rows, cols) if typ == GGML_Q4_0 else N.rand_q8_0(rng, rows, cols)
+    X = rng.normal(0, 1, (M, cols)).astype(np.float32)
+    R = rng.normal(0, 1, (M, rows)).astype(np.float32)
+    Y = _rows_gemm(P, typ, W, X, R)
+    w = N.q4_values(W) if typ == GGML_Q4_0 else N.q8_values(W)
+    w = np.asarray(w, np.float64).reshape(rows, cols)
+    prod, mag = X.astype(np.float64) @ w.T, np.abs(X).astype(np.float64) @ np.abs(w).T
+    top = np.abs(X).max(axis=1).astype(np.float64)[:, None] * np.abs(w).sum(axis=1)[None, :]
+    bound = 2.0 ** -22 * top + (cols / 8 + 8) * 2.0 ** -24 * mag + 2.0 ** -23 * (np.abs(R) + np.abs(prod))
+    assert np.all(np.abs(Y - (R + prod)) <= bound)
+
+
 def _oracle_prefill(om, prompt, L, n_ctx, kvd, flips, near=None, idx=None):
     """The oracle's prompt forward from an empty cache with the given gate
     decisions inverted: (last-token logits, K rows [L][n][kvd], V rows)."""

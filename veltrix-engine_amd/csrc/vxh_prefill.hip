@@ -6,22 +6,24 @@
 //   vx_pf_rope_kv_kernel RoPE of q|k rows and the k/v cache store (fp32 rows)
 //   vx_pf_swiglu_kernel  h = |silu(g)| < thr ? 0 : silu(g) * u
 //
-// GEMM arithmetic.  Q4_0/Q8_0 weights are d * q with q = s - 8 (resp. the
-// int8) exact in fp16 and d an fp16 scale; their product has at most 15
-// (resp. 19) significant bits, so w = w_hi + w_lo with w_hi = fp16(d q) and
-// w_lo = fp16(d q - w_hi) is exact (v_pk_fma_f16 rounds the exact remainder,
-// which fits fp16; its last bit is never below d's, 2^-24).  Activations are
-// split the same way into x_hi + x_lo.  The MFMA then accumulates
-// x_hi w_hi + x_lo w_hi + x_hi w_lo over the whole K range in fp32 -- no
-// per-block rescaling, unlike the skinny verify kernel; the dropped x_lo w_lo
-// term is below 2^-22 of each product.
+// GEMM arithmetic.  A Q4_0/Q8_0 block is d * q with q = s - 8 (resp. the int8)
+// exact in fp16 and d an fp16 scale.  Activations are split into two fp16
+// parts, x_hi + x_lo (22 bits).  Per block of 32 the MFMAs sum x_lo q and
+// x_hi q from zero, and one fp32 fma per output adds d times that block sum to
+// the running sum: two MFMA products per weight and a VALU fma that runs in
+// their shadow.  (The scheme before it folded d into the weights as an exact
+// fp16 pair and took three products, x_hi w_hi + x_lo w_hi + x_hi w_lo, with
+// no rescaling: 1.5 times the MFMA work, and its one long fp32 chain over K
+// was three times as far from the 64-bit result: 6.6e-7 against 2.3e-7 at
+// K = 4096.)
 #include "vxh_internal.h"
 #include "vxh_gemm_core.h"
 
-#define PF_BM 64                 // activation rows per workgroup
+#define PF_BM 64                 // activation rows per workgroup (a row group of the panel)
 #define PF_MT (PF_BM / 32)       // 32-row MFMA tiles per workgroup
 #define PF_STAGE (PF_MT * 2 * 2 * 2 * 64)   // A units (8 fp16) of one block pair: [mt][blk][s][hl][lane]
-#define PF_RING 3                // weight pairs in flight per wavefront
+
+typedef uint32_t vx_u32x4 __attribute__((ext_vector_type(4)));
 
 struct vx_pf_args {
     const uint4 *wq;
@@ -37,144 +39,278 @@ struct vx_pf_args {
     float scale;
 };
 
-// Workgroup = 4 wavefronts = 4 weight tiles of 32 rows (128 output columns)
-// x PF_BM activation rows.  Per block pair (64 of K) the workgroup copies the
-// activation slice of the rows panel into LDS -- MFMA A units (lane l: row
-// l%32, elements 16(l/32) + 8s .. +7 of block blk, matching the weight
-// layout's lane split), hi and lo, converted once per GEMM input by
-// vx_pf_panel_kernel instead of by each of the column workgroups (which
-// spent more VALU on it than on the weights) -- double-buffered: pair p+1 is
-// copied into the other buffer while pair p is multiplied, one barrier per
-// pair.  Each wavefront keeps
-// PF_RING pairs of its weights in flight, unpacks a pair once and runs 3
-// MFMAs per (tile, block, K half).  64-row tiles keep the grid at several
-// workgroups per CU for the 4096-column matrices of a 512-row chunk.
-template <int QT>
-__global__ __launch_bounds__(256) void vx_pf_gemm_kernel(vx_pf_args a)
+// Wavefront tile: 32 MT activation rows x 32 NT weight rows (MT = 2, or 1 in
+// a last row group of <= 32 rows).  Workgroup = CW x KS wavefronts: CW of
+// them side by side over the weight tiles, KS over the K range (block pairs
+// p with p % KS = ks), whose sums meet in LDS at the end in a fixed order.
+// Per step the workgroup copies the activation stages of its next KS pairs
+// from the rows panel into LDS (already in MFMA operand order), double-
+// buffered with one barrier per step; with CW = 1 no two wavefronts share a
+// stage and each loads its operands straight into registers.
+//
+// Bound by the matrix cores once the chip is full: 2048 x 22016 x 4096 Q4_0
+// 1742 -> 750 us (2 products: 0.98 PFLOP/s, 85% of what a large library fp16
+// product reaches here), 512 x 22016 x 4096 532 -> 241 us.  64 x 64 per
+// wavefront because an operand read from LDS then feeds two MFMAs (at 64 x 32
+// LDS reads took as long as the products); the block sums of one tile are
+// scaled and added between the MFMAs of the next, so neither pipe waits.
+template <int QT, int NT, int CW, int KS, int MT>
+__device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int cg, vx_u32x4 *lds)
 {
     constexpr int WPP = QT == 2 ? 1 : 2;
-    __shared__ uint4 lds[2 * PF_STAGE];
+    constexpr int RING = QT == 2 && CW != 2 ? 3 : 2;   // weight pairs in flight (register room)
+    constexpr bool DIRECT = CW == 1;
+    constexpr int NTHR = 64 * CW * KS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int T = blockIdx.x * 4 + wave;
-    const bool tile_ok = T < a.n_tiles;
-    const int Tc = tile_ok ? T : a.n_tiles - 1;
-    const int m0 = blockIdx.y * PF_BM;
+    const int cw = wave % CW, ks = wave / CW;
+    const int T0 = (cg * CW + cw) * NT;
     const int c = lane & 31, h = lane >> 5;
     const uint32_t magic = 0x64006400u;
-    const uint4 *wp = a.wq + (size_t)Tc * a.n_pairs * WPP * 64 + lane;
-    const uint32_t *sp = a.wd + (size_t)Tc * a.n_pairs * 32 + c;
-
-    // staging: the pair's PF_STAGE units of the rows panel, already in the
-    // LDS layout: a contiguous 16 KiB copy, 4 units per thread
-    constexpr int XU = PF_STAGE / 256;
-    const uint4 *xp = a.px + (size_t)blockIdx.y * a.n_pairs * PF_STAGE + threadIdx.x;
-    uint4 xa[XU];
-    auto load_x = [&](int p) {
+    const vx_u32x4 *wp[NT];
+    const uint32_t *sp[NT];
 #pragma unroll
-        for (int j = 0; j < XU; j++) xa[j] = xp[(size_t)p * PF_STAGE + 256 * j];
-    };
-    auto store_x = [&](uint4 *buf) {
-#pragma unroll
-        for (int j = 0; j < XU; j++) buf[threadIdx.x + 256 * j] = xa[j];
-    };
-
-    vx_f32x16 D[PF_MT];
-#pragma unroll
-    for (int mt = 0; mt < PF_MT; mt++) D[mt] = vx_f32x16{};
-    uint4 w[PF_RING][WPP];
-    uint32_t sc[PF_RING];
-#pragma unroll
-    for (int i = 0; i < PF_RING; i++) {
-        const int pi = min(i, a.n_pairs - 1);
-#pragma unroll
-        for (int q = 0; q < WPP; q++) w[i][q] = wp[((size_t)pi * WPP + q) * 64];
-        sc[i] = sp[(size_t)pi * 32];
+    for (int nt = 0; nt < NT; nt++) {
+        const int Tc = min(T0 + nt, a.n_tiles - 1);
+        wp[nt] = (const vx_u32x4 *)a.wq + (size_t)Tc * a.n_pairs * WPP * 64 + lane;
+        sp[nt] = a.wd + (size_t)Tc * a.n_pairs * 32 + c;
     }
-    load_x(0);
-    store_x(lds);
-    if (a.n_pairs > 1) load_x(1);
-    __syncthreads();
-    for (int p0 = 0; p0 < a.n_pairs; p0 += PF_RING) {
+    const vx_u32x4 *xg = (const vx_u32x4 *)a.px + (size_t)rg * a.n_pairs * PF_STAGE;
+
+    vx_u32x4 w[RING][NT][WPP];
+    uint32_t sc[RING][NT];
+    auto load_w = [&](int i, int p) {
+        const int pc = min(p, a.n_pairs - 1);
 #pragma unroll
-        for (int i = 0; i < PF_RING; i++) {
-            const int p = p0 + i;
-            if (p >= a.n_pairs) break;
-            const uint4 *cur = lds + (p & 1) * PF_STAGE;
-            // the next pair's activations into the other buffer (free since
-            // the barrier that ended pair p-1), then the one after in flight
-            if (p + 1 < a.n_pairs) {
-                store_x(lds + ((p + 1) & 1) * PF_STAGE);
-                if (p + 2 < a.n_pairs) load_x(p + 2);
-            }
-            uint4 wv[WPP];
+        for (int nt = 0; nt < NT; nt++) {
 #pragma unroll
-            for (int q = 0; q < WPP; q++) wv[q] = w[i][q];
-            const uint32_t sv = sc[i];
-            {
-                const int pn = min(p + PF_RING, a.n_pairs - 1);
+            for (int q = 0; q < WPP; q++) w[i][nt][q] = wp[nt][((size_t)pc * WPP + q) * 64];
+            sc[i][nt] = sp[nt][(size_t)pc * 32];
+        }
+    };
+    // LDS staging: XU units of a step per thread
+    constexpr int XU = DIRECT ? 1 : KS * PF_STAGE / NTHR;
+    vx_u32x4 xa[XU];
+    auto load_x = [&](int st) {
 #pragma unroll
-                for (int q = 0; q < WPP; q++) w[i][q] = wp[((size_t)pn * WPP + q) * 64];
-                sc[i] = sp[(size_t)pn * 32];
-            }
-            // weights of the pair as exact hi + lo fp16 terms
-            vx_half8 bh[2][2], bl[2][2];
+        for (int j = 0; j < XU; j++) {
+            const int u = threadIdx.x + NTHR * j;
+            const int p = min(st * KS + u / PF_STAGE, a.n_pairs - 1);
+            xa[j] = xg[(size_t)p * PF_STAGE + u % PF_STAGE];
+        }
+    };
+    auto store_x = [&](vx_u32x4 *buf) {
 #pragma unroll
-            for (int blk = 0; blk < 2; blk++) {
-                vx_half8 q0, q1;
-                if (QT == 2) {
-                    q0 = vx_unpack_q4(blk ? wv[0].z : wv[0].x, magic);
-                    q1 = vx_unpack_q4(blk ? wv[0].w : wv[0].y, magic);
-                } else {
-                    q0 = vx_unpack_q8(wv[blk].x, wv[blk].y, magic);
-                    q1 = vx_unpack_q8(wv[blk].z, wv[blk].w, magic);
+        for (int j = 0; j < XU; j++) buf[threadIdx.x + NTHR * j] = xa[j];
+    };
+    // DIRECT: the operands of one pair in registers, refilled block by block
+    vx_half8 xf[2][MT][2][2];   // [blk][mt][s][hi, lo]
+    auto load_f = [&](int blk, int p) {
+        const vx_u32x4 *xp = xg + (size_t)min(p, a.n_pairs - 1) * PF_STAGE + lane;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int hl = 0; hl < 2; hl++)
+                    xf[blk][mt][s][hl] = __builtin_bit_cast(vx_half8, xp[(((mt * 2 + blk) * 2 + s) * 2 + hl) * 64]);
+    };
+
+    vx_f32x16 acc[NT][MT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[nt][mt] = vx_f32x16{};
+    // block products of the last tile issued and the scale they wait for
+    vx_f32x16 S = vx_f32x16{};
+    float Sd = 0.0f;
+    auto add4 = [&](vx_f32x16 &P, int r0) {
+#pragma unroll
+        for (int r = r0; r < r0 + 4; r++) P[r] = fmaf(Sd, S[r], P[r]);
+    };
+    const int n_steps = (a.n_pairs + KS - 1) / KS;
+#pragma unroll
+    for (int i = 0; i < RING; i++) load_w(i, i * KS + ks);
+    if constexpr (DIRECT) {
+        load_f(0, ks);
+        load_f(1, ks);
+    } else {
+        load_x(0);
+        store_x(lds);
+        if (n_steps > 1) load_x(1);
+        __syncthreads();
+    }
+    for (int s0 = 0; s0 < n_steps; s0 += RING) {
+#pragma unroll
+        for (int i = 0; i < RING; i++) {
+            const int st = s0 + i, p = st * KS + ks;
+            if (st >= n_steps) break;
+            const vx_u32x4 *cur = lds + ((st & 1) * KS + ks) * PF_STAGE;
+            if constexpr (!DIRECT) {
+                // the next step's activations into the other buffer (free
+                // since the barrier that ended step st-1), then the one after
+                // in flight
+                if (st + 1 < n_steps) {
+                    store_x(lds + ((st + 1) & 1) * KS * PF_STAGE);
+                    if (st + 2 < n_steps) load_x(st + 2);
                 }
-                const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)((sv >> (16 * blk)) & 0xFFFFu));
-                vx_half8 dd;
-#pragma unroll
-                for (int e = 0; e < 8; e++) dd[e] = d;
-                bh[blk][0] = q0 * dd;
-                bh[blk][1] = q1 * dd;
-                bl[blk][0] = __builtin_elementwise_fma(q0, dd, -bh[blk][0]);
-                bl[blk][1] = __builtin_elementwise_fma(q1, dd, -bh[blk][1]);
             }
+            if (KS == 1 || p < a.n_pairs) {
 #pragma unroll
-            for (int blk = 0; blk < 2; blk++) {
+                for (int blk = 0; blk < 2; blk++) {
+                    vx_half8 A[MT][2][2];
 #pragma unroll
-                for (int s = 0; s < 2; s++) {
-                    vx_half8 ah[PF_MT], al[PF_MT];
+                    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                    for (int mt = 0; mt < PF_MT; mt++) {
-                        const int rest = (mt * 2 + blk) * 2 + s;
-                        ah[mt] = __builtin_bit_cast(vx_half8, cur[(rest * 2 + 0) * 64 + lane]);
-                        al[mt] = __builtin_bit_cast(vx_half8, cur[(rest * 2 + 1) * 64 + lane]);
+                        for (int s = 0; s < 2; s++)
+#pragma unroll
+                            for (int hl = 0; hl < 2; hl++)
+                                A[mt][s][hl] = DIRECT ? xf[blk][mt][s][hl]
+                                                      : __builtin_bit_cast(vx_half8, cur[(((mt * 2 + blk) * 2 + s) * 2 +
+                                                                                          hl) * 64 + lane]);
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++) {
+                        vx_half8 b0, b1;
+                        if constexpr (QT == 2) {
+                            const vx_u32x4 v = w[i][nt][0];
+                            b0 = vx_unpack_q4(blk ? v.z : v.x, magic);
+                            b1 = vx_unpack_q4(blk ? v.w : v.y, magic);
+                        } else {
+                            const vx_u32x4 v = w[i][nt][blk];
+                            b0 = vx_unpack_q8(v.x, v.y, magic);
+                            b1 = vx_unpack_q8(v.z, v.w, magic);
+                        }
+                        const float d = vx_half_bits_to_float((sc[i][nt] >> (16 * blk)) & 0xFFFFu);
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++) {
+                            // this tile's block products; the tile before it
+                            // is scaled and added in the MFMAs' shadow
+                            vx_f32x16 N = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[mt][0][1], b0, vx_f32x16{}, 0, 0, 0);
+                            const vx_half8 first = A[mt][0][1];
+                            constexpr int TILES = NT * MT;
+                            vx_f32x16 &P = acc[((nt * MT + mt + TILES - 1) % TILES) / MT][(mt + MT - 1) % MT];
+                            add4(P, 0);
+                            N = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[mt][1][1], b1, N, 0, 0, 0);
+                            add4(P, 4);
+                            N = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[mt][0][0], b0, N, 0, 0, 0);
+                            add4(P, 8);
+                            N = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[mt][1][0], b1, N, 0, 0, 0);
+                            add4(P, 12);
+                            // an MFMA that starts a chain must not write over its
+                            // own sources: keep them live past it
+                            asm volatile("" : "+v"(N) : "v"(first), "v"(b0));
+                            S = N;
+                            Sd = d;
+                        }
                     }
-#pragma unroll
-                    for (int mt = 0; mt < PF_MT; mt++)
-                        D[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[mt], bh[blk][s], D[mt], 0, 0, 0);
-#pragma unroll
-                    for (int mt = 0; mt < PF_MT; mt++)
-                        D[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[mt], bh[blk][s], D[mt], 0, 0, 0);
-#pragma unroll
-                    for (int mt = 0; mt < PF_MT; mt++)
-                        D[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[mt], bl[blk][s], D[mt], 0, 0, 0);
+                    if constexpr (DIRECT) load_f(blk, p + KS);
                 }
+                load_w(i, p + RING * KS);
             }
-            __syncthreads();
+            if constexpr (!DIRECT) __syncthreads();
         }
     }
-    const int n = T * 32 + c;
-    if (!tile_ok || n >= a.n_out) return;
+
 #pragma unroll
-    for (int mt = 0; mt < PF_MT; mt++) {
+    for (int r = 0; r < 16; r += 4) add4(acc[NT - 1][MT - 1], r);
+    const int m0 = rg * PF_BM;
+    auto put = [&](int nt, int mt, int r, float sum) {
+        const int n = (T0 + nt) * 32 + c;
+        const int row = m0 + mt * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+        if (n >= a.n_out || row >= a.M) return;
+        float v = (sum * a.rs[row]) * a.scale;   // the row scale is a power of two
+        if (a.r) v = a.r[(size_t)row * a.ldr + n] + v;
+        a.y[(size_t)row * a.ldy + n] = v;
+    };
+    if constexpr (KS == 1) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int row = m0 + mt * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-            if (row >= a.M) continue;
-            float v = (D[mt][r] * a.rs[row]) * a.scale;   // the row scale is a power of two
-            if (a.r) v = a.r[(size_t)row * a.ldr + n] + v;
-            a.y[(size_t)row * a.ldy + n] = v;
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) put(nt, mt, r, acc[nt][mt][r]);
+    } else {
+        // [ks][cw][register][lane]; the last step's barrier freed the stages
+        constexpr int R = NT * MT * 16;
+        static_assert(R % KS == 0, "registers of a tile over the K slices");
+        float *red = (float *)lds;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) red[(wave * R + (nt * MT + mt) * 16 + r) * 64 + lane] = acc[nt][mt][r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < R / KS; j++) {
+            const int reg = ks * (R / KS) + j;
+            float v = 0.0f;
+#pragma unroll
+            for (int k = 0; k < KS; k++) v += red[((k * CW + cw) * R + reg) * 64 + lane];
+            put(reg / (16 * MT), (reg / 16) % MT, reg % 16, v);
         }
     }
+}
+
+// LDS units of a workgroup: two steps' stages, or the K slices' sums
+template <int NT, int CW, int KS>
+static constexpr int vx_pf_lds_units()
+{
+    const int stage = CW == 1 ? 1 : 2 * KS * PF_STAGE, red = KS == 1 ? 0 : KS * CW * NT * PF_MT * 16 * 16;
+    return stage > red ? stage : red;
+}
+
+template <int QT, int NT, int CW, int KS>
+__global__ __launch_bounds__(64 * CW *KS, 2) void vx_pf_gemm_kernel(vx_pf_args a, int n_cg, int n_rg)
+{
+    __shared__ vx_u32x4 lds[vx_pf_lds_units<NT, CW, KS>()];
+    // workgroup id -> tile: ids go round the 8 XCDs, so every XCD takes a
+    // contiguous run of tiles, in blocks of 8 row groups: the row groups of a
+    // block share weight tiles and the columns share activation stages in L2
+    const int nb = n_cg * n_rg, x = blockIdx.x % 8, per = nb / 8, rem = nb % 8;
+    const int id = x * per + min(x, rem) + blockIdx.x / 8;
+    const int sup = id / (8 * n_cg), rs = min(8, n_rg - 8 * sup), in = id - sup * 8 * n_cg;
+    const int rg = 8 * sup + in % rs, cg = in / rs;
+    if (a.M - rg * PF_BM > 32)
+        vx_pf_gemm_body<QT, NT, CW, KS, 2>(a, rg, cg, lds);
+    else
+        vx_pf_gemm_body<QT, NT, CW, KS, 1>(a, rg, cg, lds);
+}
+
+template <int QT, int NT, int CW, int KS>
+static int vx_pf_gemm_launch(const vx_pf_args &a, hipStream_t s)
+{
+    const int n_cg = (a.n_tiles + NT * CW - 1) / (NT * CW), n_rg = (a.M + PF_BM - 1) / PF_BM;
+    vx_pf_gemm_kernel<QT, NT, CW, KS><<<(unsigned)(n_cg * n_rg), 64 * CW * KS, 0, s>>>(a, n_cg, n_rg);
+    VXH_LAUNCHED();
+    return VXH_OK;
+}
+
+// Which split: the estimated time in rounds of workgroups over the 256 CUs.
+// Each weight is the measured time of one round, in units of 40 us at
+// K = 4096 (all splits scale with K alike):
+//   64 x 256, K whole: two workgroups to a CU; a full round of 512 takes 4.05,
+//     a last one of up to 256 (one to a CU) 2.  The best rate per tile, but
+//     M = 512, N = 4096 would leave half the CUs empty.
+//   64 x 128, K over 4: 1.1 a round.  512 x 4096 x 4096 113 -> 52 us (88 with K
+//     whole); 2048 x 4096 x 4096 199 us, where K whole takes 175.
+//   64 x 64, K over 8: 0.65 a round.  512 x 2048 x 5632 148 -> 44 us (64 with
+//     64 x 128); 128 x 22016 x 4096 160 -> 71 us (85 with K whole).
+//   64 x 32, K over 8: 0.38 a round.  77 x 4096 x 11008 Q8_0 269 -> 44 us (64
+//     with 64 x 64); 48 x 4096 x 4096 103 -> 18.5 us.
+template <int QT>
+static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
+{
+    const long n_rg = (a.M + PF_BM - 1) / PF_BM;
+    auto groups = [&](int tiles) { return n_rg * ((a.n_tiles + tiles - 1) / tiles); };
+    auto rounds = [&](long n) { return (float)((n + 255) / 256); };
+    const long n0 = groups(8), rest = n0 % 512;
+    const float t0 = 4.05f * (float)(n0 / 512) + (rest == 0 ? 0.0f : rest <= 256 ? 2.0f : 4.05f);
+    const float t1 = 1.1f * rounds(groups(4)), t2 = 0.65f * rounds(groups(2)), t3 = 0.38f * rounds(groups(1));
+    const float best = fminf(fminf(t0, t1), fminf(t2, t3));
+    if (t0 == best) return vx_pf_gemm_launch<QT, 2, 4, 1>(a, s);
+    if (t1 == best) return vx_pf_gemm_launch<QT, 2, 2, 4>(a, s);
+    if (t2 == best) return vx_pf_gemm_launch<QT, 2, 1, 8>(a, s);
+    return vx_pf_gemm_launch<QT, 1, 1, 8>(a, s);
 }
 
 // Rows panel: fp32 rows x[M][ldx] as the GEMM's LDS stages.  Unit u of a
@@ -276,13 +412,7 @@ extern "C" int vxh_gemm_rows(const vxh_qmat *W, const void *px, int M, float *Y,
     a.r = R;
     a.ldr = ldr;
     a.scale = scale;
-    const dim3 grid((unsigned)((a.n_tiles + 3) / 4), (unsigned)((M + PF_BM - 1) / PF_BM));
-    if (W->type == 2)
-        vx_pf_gemm_kernel<2><<<grid, 256, 0, vxh_hs(s)>>>(a);
-    else
-        vx_pf_gemm_kernel<8><<<grid, 256, 0, vxh_hs(s)>>>(a);
-    VXH_LAUNCHED();
-    return VXH_OK;
+    return W->type == 2 ? vx_pf_gemm<2>(a, vxh_hs(s)) : vx_pf_gemm<8>(a, vxh_hs(s));
 }
 
 // ---------------------------------------------------------------------------
