@@ -568,6 +568,59 @@ def test_attention_matches_reference(P, H, KV, hd, M, n_past, n_ctx, cap):
         b.free()
 
 
+@pytest.mark.parametrize("H,KV,hd,M,n_past,n_ctx,cap", [
+    (32, 32, 64, 17, 1830, 1847, 0),      # 17 queries per kv head: one wavefront of four at work
+    (32, 32, 64, 33, 992, 1100, 0),       # a second wavefront with one query; positions end on a tile edge
+    (8, 2, 128, 97, 1200, 1500, 0),       # four query groups, the last of four queries
+    (7, 1, 128, 150, 1100, 1300, 1000),   # seven heads per kv head, cap below every row
+    (4, 4, 64, 300, 640, 940, 700),       # cap reached inside the batch
+    (4, 1, 128, 33, 8100, 8133, 0),       # segments of 16 tiles and a short last one
+    (16, 2, 64, 257, 0, 300, 0),          # empty cache: segments past the first rows' positions
+    (2, 1, 128, 600, 500, 1000, 0),       # rows past the context clamp to its last position
+    (8, 8, 128, 384, 0, 384, 0)])
+def test_prompt_attention_matches_reference(P, H, KV, hd, M, n_past, n_ctx, cap):
+    """The prompt kernel (128 queries per workgroup) against float64 softmax
+    attention, with NaN in the cache rows no query attends.  Bound: a score
+    is an fp32 sum of hd products (at most hd/4 + 8 roundings of its sum of
+    magnitudes, 2^-24 each), its exponential carries that error and 4 more
+    roundings, and each output sum rounds once per position of a tile and
+    twice per tile or segment (64 in all), relative to sum p |v|."""
+    print(f"prompt attention H={H} KV={KV} hd={hd} M={M} n_past={n_past} n_ctx={n_ctx} cap={cap}", flush=True)
+    bind_attention(P)
+    rng = np.random.default_rng(H + KV * 5 + hd + M + n_past)
+    qd, kvd = H * hd, KV * hd
+    qv = rng.normal(0, 1.0, (M, qd)).astype(np.float32)
+    kc = rng.normal(0, 1.0, (n_ctx, kvd)).astype(np.float32)
+    vc = rng.normal(0, 1.0, (n_ctx, kvd)).astype(np.float32)
+    end = min(n_past + M, n_ctx, cap or n_ctx)
+    kc[end:] = np.nan
+    vc[end:] = np.nan
+    dq, dk, dv = N.DevBuf(P, qv), N.DevBuf(P, kc), N.DevBuf(P, vc)
+    dout = N.DevBuf(P, np.zeros((M, qd), np.float32))
+    ws = Workspace()
+    assert P.vxh_workspace_alloc(C.byref(ws), 32, P.vxh_attention_workspace_floats(M, n_ctx, cap, H, KV, hd)) == 0
+    rc = P.vxh_attention(dq.ptr, M, n_past, n_ctx, H, KV, hd, cap, dk.ptr, dv.ptr, dout.ptr, qd, C.byref(ws), None)
+    assert rc == 0, P.vxh_last_error()
+    assert P.vxh_stream_sync(None) == 0
+    got = dout.get(np.float32, M * qd).reshape(M, qd)
+    P.vxh_workspace_free(C.byref(ws))
+    for b in (dq, dk, dv, dout):
+        b.free()
+    cs = np.minimum(np.minimum(n_past + np.arange(M), n_ctx - 1) + 1, cap or n_ctx)
+    dead = np.arange(end)[None, :] >= cs[:, None]
+    for h in range(H):
+        g = h // (H // KV)
+        K, Vv = (c[:end, g * hd:(g + 1) * hd].astype(np.float64) for c in (kc, vc))
+        Q = qv[:, h * hd:(h + 1) * hd].astype(np.float64)
+        s = np.where(dead, -np.inf, Q @ K.T / np.sqrt(hd))
+        mag = np.where(dead, 0.0, np.abs(Q) @ np.abs(K).T / np.sqrt(hd)).max(axis=1)
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True) + 1e-10
+        rel = 2.0 ** -24 * (2 * (hd / 4 + 8) * mag + 4 + 64)
+        bad = np.abs(got[:, h * hd:(h + 1) * hd] - p @ Vv) > rel[:, None] * (p @ np.abs(Vv))
+        assert not bad.any(), (h, np.argwhere(bad)[:4])
+
+
 def attention_ref(qv, kc, vc, H, KV, hd, n_past, n_ctx, cap):
     """Softmax attention in float64 (src/model.c:300-338): row m attends to
     [0, min(pos_m + 1, cap)), pos_m = min(n_past + m, n_ctx - 1)."""

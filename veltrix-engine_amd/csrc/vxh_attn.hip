@@ -846,6 +846,212 @@ __global__ __launch_bounds__(ATT_THREADS) __attribute__((amdgpu_waves_per_eu(3))
         q, M, n_past, n_ctx, n_heads, n_kv, cap, kc, vc, n_chunks, n_chunks_w, n_qg, part, qa);
 }
 
+// Prompt attention (many query rows from q, head_dim 64 or 128).  Workgroup =
+// (kv head, 128 query vectors, segment of the context); wavefront = 32 of the
+// queries, ordered row by row over the G heads of the kv head so that its
+// causal lengths differ by little.  K and V go through LDS in tiles of 32
+// positions, double-buffered, shared by the four wavefronts; v_mfma_f32_32x32x2
+// products with the online softmax between them.  Lane l = n + 32 h:
+//  * QK^T per (j, i): A = K[position n][8 j + 4 h + i], B = q[query n][8 j + 4 h
+//    + i]; the result holds score(position 8 (r/4) + 4 h + r % 4, query n) in
+//    item r.
+//  * P.V per (u, r): B = the probability in item r (already in place), A =
+//    V[the item's position][32 u + n]; item r of chain u is output dim
+//    32 u + 8 (r/4) + 4 h + r % 4 of query n.  A tile's sums start from zero
+//    and join the running ones with the softmax rescale in one fma, so no fp32
+//    chain is longer than a tile.
+// Bound by the fp32 matrix rate (157 TFLOP/s).  2048 rows x 32 heads of
+// 128 from an empty cache 2363 -> 458 us, 512 over 2048 positions 590 -> 193 us
+// (16-query wavefronts that each read their K and V from L2 and wrote a partial
+// per 32 positions); 500 rows x 32/4 heads of 64 over 2036 240 -> 115 us.
+#define AR_Q 128                 // query vectors per workgroup
+#define AR_T 32                  // positions per tile
+
+// e^x for x <= 0 (NaN stays NaN): 2^(x log2 e) with the product's rounding
+// error e carried in a first-order term; below e^-150 (0 in fp32) it is 0.
+__device__ __forceinline__ float vx_exp_neg(float x)
+{
+    x = x < -150.0f ? -150.0f : x;
+    const float L = 1.44269502f, L_LO = 1.92596303e-8f;    // log2 e in two parts
+    const float t = x * L;
+    const float e = fmaf(x, L_LO, fmaf(x, L, -t));
+    const float r = __builtin_amdgcn_exp2f(t);
+    return fmaf(r, e * 0.693147181f, r);
+}
+
+template <int HD>
+__global__ __launch_bounds__(256, 2) void vx_attention_rows_kernel(
+    const float *__restrict__ q, int M, int n_past, int n_ctx, int n_heads, int n_kv, int cap,
+    const float *__restrict__ kc, const float *__restrict__ vc, int n_qg, int n_seg, int seg_len,
+    float *__restrict__ part, float *__restrict__ out, int ld_out)
+{
+    // row strides: 4 floats of padding spread a K column's rows over the
+    // banks; 8 put the two lane halves' V rows (4 apart) on other banks
+    constexpr int KS = HD + 4, VS = HD + 8, NU = HD / 32, NJ = HD / 8;
+    constexpr int X4 = AR_T * HD / 4 / 256;      // float4 per thread of a K or V tile
+    __shared__ float s_k[2][AR_T * KS], s_v[2][AR_T * VS];
+    // kv heads go round the XCDs (8 or more: a head's K and V stay in one L2)
+    const int g = blockIdx.x % n_kv, rest = blockIdx.x / n_kv;
+    const int seg = rest / n_qg, qg = n_qg - 1 - rest % n_qg;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    const int G = n_heads / n_kv, QM = G * M, kvd = n_kv * HD;
+
+    auto causal = [&](int m) {
+        const int len = min(n_past + m, n_ctx - 1) + 1;
+        return cap > 0 && len > cap ? cap : len;
+    };
+    const int qi = qg * AR_Q + wave * 32 + n;
+    const bool qok = qi < QM;
+    const int m = qok ? qi / G : 0, head = g * G + (qok ? qi % G : 0);
+    const int cs = qok ? causal(m) : 0;
+    float *pq = part + (((size_t)g * n_seg + seg) * QM + (size_t)(head - g * G) * M + m) * PART_STRIDE(HD);
+    const int t_begin = seg * seg_len;
+    const int t_end = min(t_begin + seg_len, causal(min(M - 1, (qg * AR_Q + AR_Q - 1) / G)));
+    if (t_begin >= t_end) {        // a segment past these queries' positions
+        if (qok && h == 0 && n_seg > 1) {
+            pq[0] = -INFINITY;
+            pq[1] = 0.0f;
+        }
+        return;
+    }
+    // the wavefront's own range: all of its queries reach lo, none passes hi
+    const int q0 = qg * AR_Q + wave * 32;
+    const int lo = __builtin_amdgcn_readfirstlane(causal(min(q0 / G, M - 1)));
+    const int hi = __builtin_amdgcn_readfirstlane(q0 < QM ? causal(min((q0 + 31) / G, M - 1)) : 0);
+
+    const float scale = 1.0f / sqrtf((float)HD);
+    vx_f32x4 qv[NJ];
+    {
+        const float *qr = q + (size_t)m * n_heads * HD + (size_t)head * HD + 4 * h;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) qv[j] = *(const vx_f32x4 *)(qr + 8 * j) * (qok ? scale : 0.0f);
+    }
+
+    vx_f32x4 st[X4];
+    auto load = [&](const float *c, int t) {
+#pragma unroll
+        for (int i = 0; i < X4; i++) {
+            const int u = threadIdx.x + 256 * i, row = u / (HD / 4), d4 = u % (HD / 4);
+            const int pos = min(t + row, n_ctx - 1);
+            st[i] = *(const vx_f32x4 *)(c + (size_t)pos * kvd + g * HD + 4 * d4);
+        }
+    };
+    auto store = [&](float *b, int stride, int t) {
+#pragma unroll
+        for (int i = 0; i < X4; i++) {
+            const int u = threadIdx.x + 256 * i, row = u / (HD / 4), d4 = u % (HD / 4);
+            // rows no query attends are zeros: 0 times what a cache holds there may be NaN
+            *(vx_f32x4 *)(b + row * stride + 4 * d4) = t + row < t_end ? st[i] : vx_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    load(kc, t_begin);
+    store(s_k[0], KS, t_begin);
+    load(vc, t_begin);
+    store(s_v[0], VS, t_begin);
+    __syncthreads();
+
+    vx_f32x16 O[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) O[u] = vx_f32x16{};
+    float rm = -INFINITY, rl = 0.0f;
+    for (int t = t_begin, b = 0; t < t_end; t += AR_T, b ^= 1) {
+        const bool more = t + AR_T < t_end;
+        const bool live = t < hi;      // uniform over the wavefront
+        if (more) load(kc, t + AR_T);
+        vx_f32x16 S;
+        if (live) {
+            // two chains, so that no sum runs over more than half a head
+            vx_f32x16 S1;
+            const float *kb = s_k[b] + n * KS + 4 * h;
+            vx_f32x4 k0, k1;
+#pragma unroll
+            for (int j = 0; j < NJ; j += 2) {
+                const vx_f32x4 ka = *(const vx_f32x4 *)(kb + 8 * j), kd = *(const vx_f32x4 *)(kb + 8 * j + 8);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    S = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[i], qv[j][i], j + i == 0 ? vx_f32x16{} : S, 0, 0, 0);
+                    S1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[i], qv[j + 1][i], j + i == 0 ? vx_f32x16{} : S1, 0, 0,
+                                                              0);
+                }
+                if (j == 0) {
+                    k0 = ka;
+                    k1 = kd;
+                }
+            }
+            // an MFMA that starts a chain must not write over its own sources
+            asm volatile("" : "+v"(S), "+v"(S1) : "v"(k0), "v"(k1));
+            S += S1;
+        }
+        if (more) {
+            store(s_k[b ^ 1], KS, t + AR_T);
+            load(vc, t + AR_T);
+        }
+        if (live) {
+            float cm = -INFINITY;
+            if (t + AR_T > lo) {
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (t + 8 * (r / 4) + 4 * h + r % 4 >= cs) S[r] = -INFINITY;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) cm = fmaxf(cm, S[r]);
+            cm = vx_max_x32(cm);
+            const float nm = fmaxf(rm, cm);
+            const float base = nm == -INFINITY ? 0.0f : nm;    // -inf scores: probability 0
+            const float fo = vx_exp_neg(rm - base);
+            float l = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                S[r] = vx_exp_neg(S[r] - base);
+                l += S[r];
+            }
+            rl = fmaf(rl, fo, l);                               // this half's positions
+            rm = nm;
+            const float *vb = s_v[b] + 4 * h * VS + n;
+#pragma unroll
+            for (int u = 0; u < NU; u += 2) {
+                vx_f32x16 T[2];
+                float v0[2];
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+#pragma unroll
+                    for (int w = 0; w < 2; w++) {
+                        const float v = vb[(8 * (r / 4) + r % 4) * VS + 32 * (u + w)];
+                        T[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, S[r], r == 0 ? vx_f32x16{} : T[w], 0, 0, 0);
+                        if (r == 0) v0[w] = v;
+                    }
+                asm volatile("" : "+v"(T[0]), "+v"(T[1]) : "v"(v0[0]), "v"(v0[1]), "v"(S[0]));
+#pragma unroll
+                for (int w = 0; w < 2; w++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) O[u + w][r] = fmaf(O[u + w][r], fo, T[w][r]);
+            }
+        }
+        if (more) store(s_v[b ^ 1], VS, t + AR_T);
+        __syncthreads();
+    }
+    rl = vx_sum_x32(rl);
+    if (!qok) return;
+    float *o;
+    float f = 1.0f;
+    if (n_seg > 1) {
+        if (h == 0) {
+            pq[0] = rm;
+            pq[1] = rl;
+        }
+        o = pq + 4;
+    } else {
+        o = out + (size_t)m * ld_out + (size_t)head * HD;
+        f = 1.0f / (rl + 1e-10f);
+    }
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            *(vx_f32x4 *)(o + 32 * u + 8 * i + 4 * h) =
+                vx_f32x4{O[u][4 * i] * f, O[u][4 * i + 1] * f, O[u][4 * i + 2] * f, O[u][4 * i + 3] * f};
+}
+
 // One workgroup per (row m, head): merge the chunks' partial results with
 // the online-softmax rescale and normalise by 1/(sum + 1e-10)
 // (src/tensor.c:156-171).  Thread t owns float4 lane d4 = t % (hd/4) of the
@@ -987,6 +1193,31 @@ static void vx_attention_mfma_launch(const float *q, bool qkv, const vx_qkv_args
             q, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
 }
 
+static int vx_attention_combine(const float *part, int M, int n_heads, int n_kv_heads, int head_dim, int n_chunks,
+                                float *out, int ld_out, double *clr, long n_clr, vxh_stream s)
+{
+    const int per = (n_chunks + CMB_THREADS / (head_dim / 4) - 1) / (CMB_THREADS / (head_dim / 4));
+#define VX_CMB_LAUNCH(NB_)                                                                                      \
+    vx_attention_combine_kernel<NB_><<<M * n_heads, CMB_THREADS, 0, vxh_hs(s)>>>(                               \
+        part, M, n_heads, n_kv_heads, head_dim, n_chunks, out, ld_out, clr, n_clr)
+    if (per <= 4) VX_CMB_LAUNCH(4);
+    else if (per <= 6) VX_CMB_LAUNCH(6);
+    else if (per <= 8) VX_CMB_LAUNCH(8);
+    else VX_CMB_LAUNCH(12);
+#undef VX_CMB_LAUNCH
+    VXH_LAUNCHED();
+    return VXH_OK;
+}
+
+// Scores (heads x rows x positions) from which the prompt kernel takes q rows.
+// Below it 16-query wavefronts of one chunk each spread the little work over
+// more CUs (48 rows x 32 heads of 128 over 148 positions: 15.0 us there, 16.6
+// here; 100 x 8 x 64 over 600: 13.5 and 14.9); from it the prompt kernel is as
+// fast or faster (20 x 32 x 128 over 2020: 42.5 and 40.0; 100 x 32 x 128 over
+// 1100: 86 and 48).  Batches that the q|k|v kernel also takes (at most
+// VX_ATT_MFMA_MAX_M rows) keep its order of sums at any size.
+#define VX_ROWS_MIN_SCORES 1e6
+
 // parts_only: the first launch alone; the partials stay in ws->part for a
 // consumer that combines them itself (*n_chunks_out chunks per query).
 static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, int M, int n_past,
@@ -1021,6 +1252,33 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     size_t need = (size_t)n_kv_heads * n_chunks * QM * PART_STRIDE(head_dim);
     if (need > ws->part_floats)
         return vxh_fail(VXH_ERR_PARAM, "attention workspace too small (%zu floats needed)", need);
+    const bool rows = !qa && !parts_only && (head_dim == 64 || head_dim == 128) && M > VX_ATT_MFMA_MAX_M &&
+                      (double)n_heads * M * ctx >= VX_ROWS_MIN_SCORES;
+    if (rows) {
+        // segments of whole tiles: about two workgroups per CU in all
+        const int nqg = (QM + AR_Q - 1) / AR_Q, n_t = (ctx + AR_T - 1) / AR_T;
+        const long wgs = (long)n_kv_heads * nqg;
+        // 512 workgroups (two per CU) once a CU has 8 tiles or more to do, else 256:
+        // 500 rows x 32 heads of 64 over 2036 positions 122 us at 256, 115 at 512;
+        // 100 rows x 32 heads of 128 over 1100: 48 and 50.  At most 1024 positions a
+        // segment: the workgroups of a long causal prompt end together.
+        const long target = wgs * n_t >= 2048 ? 512 : 256;
+        int n_seg = (int)((target + wgs - 1) / wgs);
+        if (n_seg < (n_t + 31) / 32) n_seg = (n_t + 31) / 32;
+        if (n_seg > n_t) n_seg = n_t;
+        const int seg_t = (n_t + n_seg - 1) / n_seg;
+        n_seg = (n_t + seg_t - 1) / seg_t;
+        const unsigned grid = (unsigned)(wgs * n_seg);
+        if (head_dim == 64)
+            vx_attention_rows_kernel<64><<<grid, 256, 0, vxh_hs(s)>>>(q, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc,
+                                                                     nqg, n_seg, seg_t * AR_T, ws->part, out, ld_out);
+        else
+            vx_attention_rows_kernel<128><<<grid, 256, 0, vxh_hs(s)>>>(q, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc,
+                                                                      nqg, n_seg, seg_t * AR_T, ws->part, out, ld_out);
+        VXH_LAUNCHED();
+        if (n_seg == 1) return VXH_OK;
+        return vx_attention_combine(ws->part, M, n_heads, n_kv_heads, head_dim, n_seg, out, ld_out, nullptr, 0, s);
+    }
     size_t lds = vx_attn_lds(qpg, head_dim);
     vx_qkv_args none;
     memset(&none, 0, sizeof(none));
@@ -1064,17 +1322,7 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     if (n_chunks_out) *n_chunks_out = n_chunks;
     if (parts_only) return VXH_OK;
     double *clr = (qa && n_clr > 0) ? (double *)qa->qkv : nullptr;
-    const int per = (n_chunks + CMB_THREADS / (head_dim / 4) - 1) / (CMB_THREADS / (head_dim / 4));
-#define VX_CMB_LAUNCH(NB_)                                                                                      \
-    vx_attention_combine_kernel<NB_><<<M * n_heads, CMB_THREADS, 0, vxh_hs(s)>>>(                               \
-        ws->part, M, n_heads, n_kv_heads, head_dim, n_chunks, out, ld_out, clr, n_clr)
-    if (per <= 4) VX_CMB_LAUNCH(4);
-    else if (per <= 6) VX_CMB_LAUNCH(6);
-    else if (per <= 8) VX_CMB_LAUNCH(8);
-    else VX_CMB_LAUNCH(12);
-#undef VX_CMB_LAUNCH
-    VXH_LAUNCHED();
-    return VXH_OK;
+    return vx_attention_combine(ws->part, M, n_heads, n_kv_heads, head_dim, n_chunks, out, ld_out, clr, n_clr, s);
 }
 
 extern "C" int vxh_attention(const float *q, int M, int n_past, int n_ctx, int n_heads,
