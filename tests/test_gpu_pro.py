@@ -568,6 +568,37 @@ def test_attention_matches_reference(P, H, KV, hd, M, n_past, n_ctx, cap):
         b.free()
 
 
+@pytest.mark.parametrize("H,KV,hd,M", [(3, 1, 32, 1), (3, 3, 32, 2), (5, 1, 32, 1)])
+@pytest.mark.parametrize("after", [1e30, np.inf, np.nan])
+def test_pro_attn_reads_no_head_past_k(P, H, KV, hd, M, after):
+    """An odd number of 32-column blocks: the attention prologue's last block
+    pair ends past the heads, and what lies after the partials must reach
+    neither the row scale nor a sum.  One chunk per query, so the combined
+    row is acc / (sum + 1e-10)."""
+    print(f"gemm_pro attn past K H={H} KV={KV} hd={hd} M={M} after={after}", flush=True)
+    bind_attention(P)
+    rng = np.random.default_rng(H * 7 + KV + M)
+    K, G, ps = H * hd, H // KV, hd + 4
+    W = rand_w(rng, 2, 64, K)
+    q = qmat(P, W, 2)
+    part = np.full((2 * KV + 2, G * M, ps), after, np.float32)      # [kv head][query hl * M + m][max, sum, -, -, acc]
+    part[:KV, :, 0] = 0.0
+    part[:KV, :, 1] = rng.uniform(1.0, 4.0, (KV, G * M))
+    part[:KV, :, 4:] = rng.normal(0, 1, (KV, G * M, hd))
+    dpart = N.DevBuf(P, part)
+    x = (part[:KV, :, 4:].astype(np.float64) / (part[:KV, :, 1:2].astype(np.float64) + 1e-10))
+    x = x.reshape(KV, G, M, hd).transpose(2, 0, 1, 3).reshape(M, K)
+    pro = Pro(kind=PRO_ATTN, part=dpart.ptr, n_chunks=1, n_heads=H, n_kv_heads=KV, head_dim=hd)
+    acc = run_pro(P, q, M, pro, 64, 64)
+    got = acc.get(np.float64, M * 64).reshape(M, 64)
+    ref, exact = oracle_gemv(W, 2, x.astype(np.float32))
+    ok, _ = N.parity(got, ref, exact)
+    assert ok, max_violation(got, ref)
+    dpart.free()
+    acc.free()
+    P.vxh_qmat_free(C.byref(q))
+
+
 @pytest.mark.parametrize("H,KV,hd,M,n_past,n_ctx,cap", [
     (32, 32, 64, 17, 1830, 1847, 0),      # 17 queries per kv head: one wavefront of four at work
     (32, 32, 64, 33, 992, 1100, 0),       # a second wavefront with one query; positions end on a tile edge

@@ -271,8 +271,10 @@ __device__ __forceinline__ void vx_pro_attn(const vx_pro_args &p, int p0, int np
     const int m = u / L4, c4 = u % L4;
     float mx = -INFINITY, l = 0.0f;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (sl < S) {
-        const int e = k0 + 4 * c4;
+    const int e = k0 + 4 * c4;
+    // columns past K (an odd block count) have no head: zeros, not the memory
+    // after the partials, whose magnitude would set the row's scale
+    if (sl < S && e < p.K) {
         const int head = e / hd, d4 = (e % hd) / 4;
         const int g = head / p.G, qi = (head % p.G) * M + m;
         const float *pq = p.part + (size_t)g * p.n_chunks * cstride + (size_t)qi * PS;
