@@ -59,7 +59,7 @@ typedef struct {
                                   then hold halves                                    */
     int prefill_min_rows;      /* prompt chunks of at least this many rows whose
                                   positions fit the context run as one large-M
-                                  batch (up to 512 rows; exact Q4_0 kernel, fp32
+                                  batch (up to 2048 rows; exact Q4_0 kernel, fp32
                                   cache); 0 = never.  Default 48               */
 } vx_model_options;
 

@@ -459,6 +459,15 @@ int vxh_attention_parts_qkv_f16(double *qkv, int ld_qkv, const double *ss, int s
 
 size_t vxh_attention_workspace_floats(int M, int n_ctx, int cap, int n_heads, int n_kv_heads,
                                       int head_dim);
+/* vxh_attention on a workspace of vxh_attention_rows_workspace_floats(M, ...)
+ * floats, enough for any batch of up to M rows: long batches keep a partial
+ * per context segment instead of one per 32 positions (2048 rows x 32 heads of
+ * 128 over 32768 positions: 1.1 GB instead of 35). */
+int vxh_attention_rows(const float *q, int M, int n_past, int n_ctx, int n_heads, int n_kv_heads, int head_dim,
+                       int cap, const float *k_cache_layer, const float *v_cache_layer, float *out, int ld_out,
+                       vxh_workspace *ws, vxh_stream s);
+size_t vxh_attention_rows_workspace_floats(int M, int n_ctx, int cap, int n_heads, int n_kv_heads,
+                                           int head_dim);
 
 /* ---- elementwise ------------------------------------------------------------- */
 /* y[m][i] += x[m][i] for i < n (residual add, src/model.c:546, :589). */

@@ -109,6 +109,37 @@ def test_prefill_matches_oracle(P, tmp_path, case):
     assert close(ver, vref), max_violation(ver, vref)
 
 
+@pytest.mark.parametrize("d,h,kv", [(256, 4, 2), (256, 2, 1), (192, 2, 1)])
+def test_prefill_buffers_grow(P, tmp_path, d, h, kv):
+    """Prompts of 60, 1300 and 2100 rows in turn on one model (the prefill
+    buffers grow; 2100 is more than one chunk; at head_dim 96 the chunks stay
+    at 512 rows): logits and cached rows as the batched decode forward gives
+    them (fp32 bar)."""
+    print(f"prefill growth d{d} {h}/{kv}", flush=True)
+    rng = np.random.default_rng(d + h)
+    path = str(tmp_path / "m.gguf")
+    V, n_ctx, kvd = 64, 2200, kv * (d // h)
+    llama_gguf(path, rng, 1, d, h, kv, 256, V, std=0.05, norm_random=True, emb_type=GGML_Q4_0, out_type=GGML_Q4_0,
+               matrix_type=GGML_Q4_0)
+    mp, mb = load(P, path, n_ctx), load(P, path, n_ctx, prefill_min_rows=0)
+    try:
+        for n in (60, 1300, 2100):
+            prompt = rng.integers(0, V, n).astype(np.int32)
+            out = []
+            for m in (mp, mb):
+                P.vx_model_kv_truncate(m, 0)
+                lg, k, v = np.zeros(V, np.float32), np.zeros((n, kvd), np.float32), np.zeros((n, kvd), np.float32)
+                assert P.vx_model_forward(m, prompt, n, lg) == 0, N.product_error()
+                assert m.contents.cache_len == n
+                assert P.vx_model_read_kv(m, 0, n, k, v) == 0, N.product_error()
+                out.append((lg, k, v))
+            for got, ref in zip(*out):
+                assert close(got, ref), (n, max_violation(got, ref))
+    finally:
+        P.vx_model_destroy(mp)
+        P.vx_model_destroy(mb)
+
+
 def _rows_gemm(P, typ, W, X, R=None, scale=1.0):
     """vxh_rows_panel + vxh_gemm_rows on host arrays: Y = R + scale X W^T."""
     vp = C.c_void_p

@@ -1161,6 +1161,51 @@ extern "C" size_t vxh_attention_workspace_floats(int M, int n_ctx, int cap, int 
     return (size_t)n_kv_heads * n_chunks * (n_heads / n_kv_heads) * M * PART_STRIDE(head_dim);
 }
 
+// Scores (heads x rows x positions) from which the prompt kernel takes q rows.
+// Below it 16-query wavefronts of one chunk each spread the little work over
+// more CUs (48 rows x 32 heads of 128 over 148 positions: 15.0 us there, 16.6
+// here; 100 x 8 x 64 over 600: 13.5 and 14.9); from it the prompt kernel is as
+// fast or faster (20 x 32 x 128 over 2020: 42.5 and 40.0; 100 x 32 x 128 over
+// 1100: 86 and 48).  Batches that the q|k|v kernel also takes (at most
+// VX_ATT_MFMA_MAX_M rows) keep its order of sums at any size.
+#define VX_ROWS_MIN_SCORES 1e6
+
+// Context segments of the prompt kernel, in whole tiles (*seg_t of them each):
+// 512 workgroups (two per CU) once a CU has 8 tiles or more to do, else 256:
+// 500 rows x 32 heads of 64 over 2036 positions 122 us at 256, 115 at 512;
+// 100 rows x 32 heads of 128 over 1100: 48 and 50.  At most 1024 positions a
+// segment: the workgroups of a long causal prompt end together.
+static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int *seg_t)
+{
+    const int n_t = (ctx + AR_T - 1) / AR_T;
+    const long wgs = (long)n_kv_heads * ((QM + AR_Q - 1) / AR_Q), target = wgs * n_t >= 2048 ? 512 : 256;
+    int n_seg = (int)((target + wgs - 1) / wgs);
+    if (n_seg < (n_t + 31) / 32) n_seg = (n_t + 31) / 32;
+    if (n_seg > n_t) n_seg = n_t;
+    *seg_t = (n_t + n_seg - 1) / n_seg;
+    return (n_t + *seg_t - 1) / *seg_t;
+}
+
+// What any batch of up to M rows over up to ctx positions needs: the chunk
+// kernels' partials where they run (VX_ATT_MFMA_MAX_M rows, or fewer scores
+// than VX_ROWS_MIN_SCORES), the segments' elsewhere (at most 128 queries for
+// each of 512 workgroups and one more segment, or 1024 positions a segment).
+extern "C" size_t vxh_attention_rows_workspace_floats(int M, int n_ctx, int cap, int n_heads, int n_kv_heads,
+                                                      int head_dim)
+{
+    const size_t full = vxh_attention_workspace_floats(M, n_ctx, cap, n_heads, n_kv_heads, head_dim);
+    if (head_dim != 64 && head_dim != 128) return full;
+    const size_t ctx = cap > 0 && n_ctx > cap ? cap : n_ctx, q = (size_t)n_heads * M;
+    const size_t few = (size_t)n_heads * VX_ATT_MFMA_MAX_M * ((ctx + ACH - 1) / ACH);
+    const size_t small = (size_t)(VX_ROWS_MIN_SCORES / ACH) + 1 + q;
+    const size_t seg = 512 * AR_Q + q, lon = q * ((ctx + 1023) / 1024 + 1);
+    size_t need = few > small ? few : small;
+    if (seg > need) need = seg;
+    if (lon > need) need = lon;
+    need *= PART_STRIDE(head_dim);
+    return need < full ? need : full;
+}
+
 // a layer's attended cache rows beyond this many bytes are read with
 // non-temporal loads
 #define VX_KV_STREAM_BYTES (16.0 * 1024 * 1024)
@@ -1209,22 +1254,14 @@ static int vx_attention_combine(const float *part, int M, int n_heads, int n_kv_
     return VXH_OK;
 }
 
-// Scores (heads x rows x positions) from which the prompt kernel takes q rows.
-// Below it 16-query wavefronts of one chunk each spread the little work over
-// more CUs (48 rows x 32 heads of 128 over 148 positions: 15.0 us there, 16.6
-// here; 100 x 8 x 64 over 600: 13.5 and 14.9); from it the prompt kernel is as
-// fast or faster (20 x 32 x 128 over 2020: 42.5 and 40.0; 100 x 32 x 128 over
-// 1100: 86 and 48).  Batches that the q|k|v kernel also takes (at most
-// VX_ATT_MFMA_MAX_M rows) keep its order of sums at any size.
-#define VX_ROWS_MIN_SCORES 1e6
-
 // parts_only: the first launch alone; the partials stay in ws->part for a
 // consumer that combines them itself (*n_chunks_out chunks per query).
+// rows_ws: ws is sized by vxh_attention_rows_workspace_floats.
 static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, int M, int n_past,
                             int n_ctx, int n_heads, int n_kv_heads, int head_dim, int cap, float *kc,
                             float *vc, float *out, int ld_out, vxh_workspace *ws,
                             int parts_only, int *n_chunks_out,
-                            vxh_stream s, int kv_half = 0)
+                            vxh_stream s, int kv_half = 0, bool rows_ws = false)
 {
     if (kv_half && (!qa || (head_dim != 64 && head_dim != 128) || M > VX_ATT_MFMA_MAX_M))
         return vxh_fail(VXH_ERR_UNSUPPORTED, "attention: an fp16 KV cache needs the q|k|v kernel, head_dim "
@@ -1249,26 +1286,16 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     int qpg = vx_attn_qpg(head_dim);
     if (qpg > QM) qpg = QM;
     int n_qg = (QM + qpg - 1) / qpg;
-    size_t need = (size_t)n_kv_heads * n_chunks * QM * PART_STRIDE(head_dim);
-    if (need > ws->part_floats)
-        return vxh_fail(VXH_ERR_PARAM, "attention workspace too small (%zu floats needed)", need);
     const bool rows = !qa && !parts_only && (head_dim == 64 || head_dim == 128) && M > VX_ATT_MFMA_MAX_M &&
                       (double)n_heads * M * ctx >= VX_ROWS_MIN_SCORES;
+    int seg_t = 0;
+    const int n_seg = rows ? vx_rows_segments(n_kv_heads, QM, ctx, &seg_t) : 0;
+    size_t need = (size_t)n_kv_heads * (rows && rows_ws ? n_seg : n_chunks) * QM * PART_STRIDE(head_dim);
+    if (need > ws->part_floats)
+        return vxh_fail(VXH_ERR_PARAM, "attention workspace too small (%zu floats needed)", need);
     if (rows) {
-        // segments of whole tiles: about two workgroups per CU in all
-        const int nqg = (QM + AR_Q - 1) / AR_Q, n_t = (ctx + AR_T - 1) / AR_T;
-        const long wgs = (long)n_kv_heads * nqg;
-        // 512 workgroups (two per CU) once a CU has 8 tiles or more to do, else 256:
-        // 500 rows x 32 heads of 64 over 2036 positions 122 us at 256, 115 at 512;
-        // 100 rows x 32 heads of 128 over 1100: 48 and 50.  At most 1024 positions a
-        // segment: the workgroups of a long causal prompt end together.
-        const long target = wgs * n_t >= 2048 ? 512 : 256;
-        int n_seg = (int)((target + wgs - 1) / wgs);
-        if (n_seg < (n_t + 31) / 32) n_seg = (n_t + 31) / 32;
-        if (n_seg > n_t) n_seg = n_t;
-        const int seg_t = (n_t + n_seg - 1) / n_seg;
-        n_seg = (n_t + seg_t - 1) / seg_t;
-        const unsigned grid = (unsigned)(wgs * n_seg);
+        const int nqg = (QM + AR_Q - 1) / AR_Q;
+        const unsigned grid = (unsigned)((long)n_kv_heads * nqg * n_seg);
         if (head_dim == 64)
             vx_attention_rows_kernel<64><<<grid, 256, 0, vxh_hs(s)>>>(q, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc,
                                                                      nqg, n_seg, seg_t * AR_T, ws->part, out, ld_out);
@@ -1332,6 +1359,14 @@ extern "C" int vxh_attention(const float *q, int M, int n_past, int n_ctx, int n
 {
     return vx_attention_run(q, nullptr, 0, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap,
                             (float *)kc, (float *)vc, out, ld_out, ws, 0, nullptr, s);
+}
+
+extern "C" int vxh_attention_rows(const float *q, int M, int n_past, int n_ctx, int n_heads, int n_kv_heads,
+                                  int head_dim, int cap, const float *kc, const float *vc, float *out, int ld_out,
+                                  vxh_workspace *ws, vxh_stream s)
+{
+    return vx_attention_run(q, nullptr, 0, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap,
+                            (float *)kc, (float *)vc, out, ld_out, ws, 0, nullptr, s, 0, true);
 }
 
 static int vx_attention_qkv(double *qkv, int ld_qkv, const double *ss, int ss_K, const float *bq,

@@ -55,8 +55,10 @@ extern "C" int vxh_malloc(void **p, size_t bytes)
     *p = nullptr;
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not by the next launch
         return vxh_fail(VXH_ERR_ALLOC, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    }
     return VXH_OK;
 }
 

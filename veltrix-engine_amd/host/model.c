@@ -158,6 +158,17 @@ static int gu_rows(int F) { return (F + 15) / 16 * 32; }
 static int round32(int n) { return (n + 31) / 32 * 32; }
 static void prof_free(vx_dev *d);
 
+static void pf_free(vx_dev *d)
+{
+    vxh_free(d->pf_tok); vxh_free(d->pf_x); vxh_free(d->pf_xn); vxh_free(d->pf_qkv);
+    vxh_free(d->pf_q); vxh_free(d->pf_att); vxh_free(d->pf_gu); vxh_free(d->pf_h); vxh_free(d->pf_px);
+    d->pf_tok = NULL;
+    d->pf_x = d->pf_xn = d->pf_qkv = d->pf_q = d->pf_att = d->pf_gu = d->pf_h = NULL;
+    d->pf_px = NULL;
+    vxh_workspace_free(&d->pf_ws);
+    d->pf_rows = 0;
+}
+
 static void dev_free(vx_dev *d)
 {
     if (!d) return;
@@ -180,9 +191,7 @@ static void dev_free(vx_dev *d)
     vxh_free(d->stats); vxh_free(d->acc_out);
     vxh_free(d->ss);
     vxh_free(d->x2); vxh_free(d->acc_y);
-    vxh_free(d->pf_tok); vxh_free(d->pf_x); vxh_free(d->pf_xn); vxh_free(d->pf_qkv);
-    vxh_free(d->pf_q); vxh_free(d->pf_att); vxh_free(d->pf_gu); vxh_free(d->pf_h); vxh_free(d->pf_px);
-    vxh_workspace_free(&d->pf_ws);
+    pf_free(d);
     vxh_panel_free(&d->pan_d);
     vxh_panel_free(&d->pan_f);
     vxh_workspace_free(&d->ws);
@@ -1153,21 +1162,19 @@ static int pf_ok(const vx_dev *d)
            !d->has_f32 && d->hd % 4 == 0 && d->hd <= 128;
 }
 
-static vx_error pf_alloc(vx_dev *d)
+static vx_error pf_ws_alloc(vx_dev *d, int R)
 {
-    if (d->pf_ready && (d->pf_ws_ctx != d->n_ctx_alloc || d->pf_ws_cap != d->opt.attn_cap)) {
-        /* a cache allocated again for another n_ctx, or another cap: the
-         * attention workspace is sized for both */
-        TRY(vxh_stream_sync(d->stream));
-        vxh_workspace_free(&d->pf_ws);
-        size_t an = vxh_attention_workspace_floats(VX_PF_ROWS, d->n_ctx_alloc, d->opt.attn_cap, d->n_heads,
-                                                   d->n_kv, d->hd);
-        TRY(vxh_workspace_alloc(&d->pf_ws, 32, an));
-        d->pf_ws_ctx = d->n_ctx_alloc;
-        d->pf_ws_cap = d->opt.attn_cap;
-    }
-    if (d->pf_ready) return VX_OK;
-    const size_t R = VX_PF_ROWS;
+    TRY(vxh_workspace_alloc(&d->pf_ws, 32,
+                            vxh_attention_rows_workspace_floats(R, d->n_ctx_alloc, d->opt.attn_cap, d->n_heads,
+                                                                d->n_kv, d->hd)));
+    d->pf_ws_ctx = d->n_ctx_alloc;
+    d->pf_ws_cap = d->opt.attn_cap;
+    return VX_OK;
+}
+
+static vx_error pf_alloc_rows(vx_dev *d, int rows)
+{
+    const size_t R = rows;
     TRY(vxh_malloc((void **)&d->pf_tok, sizeof(int) * R));
     TRY(vxh_malloc((void **)&d->pf_x, sizeof(float) * R * d->d));
     TRY(vxh_malloc((void **)&d->pf_xn, sizeof(float) * R * d->d));
@@ -1176,17 +1183,41 @@ static vx_error pf_alloc(vx_dev *d)
     TRY(vxh_malloc((void **)&d->pf_att, sizeof(float) * R * d->d));
     TRY(vxh_malloc((void **)&d->pf_gu, sizeof(float) * R * d->ld_gu));
     TRY(vxh_malloc((void **)&d->pf_h, sizeof(float) * R * d->F));
-    TRY(vxh_malloc((void **)&d->pf_px, vxh_rows_panel_bytes(VX_PF_ROWS, d->F > d->d ? d->F : d->d)));
-    size_t an = vxh_attention_workspace_floats(VX_PF_ROWS, d->n_ctx_alloc, d->opt.attn_cap, d->n_heads, d->n_kv,
-                                               d->hd);
-    TRY(vxh_workspace_alloc(&d->pf_ws, 32, an));
-    d->pf_ws_ctx = d->n_ctx_alloc;
-    d->pf_ws_cap = d->opt.attn_cap;
-    d->pf_ready = 1;
-    return VX_OK;
+    TRY(vxh_malloc(&d->pf_px, vxh_rows_panel_bytes(rows, d->F > d->d ? d->F : d->d)));
+    vx_error e = pf_ws_alloc(d, rows);
+    if (e == VX_OK) d->pf_rows = rows;
+    return e;
 }
 
-/* M <= VX_PF_ROWS prompt rows at positions n_past .. n_past+M-1 (all below
+/* Buffers for a chunk of P rows (grown in steps of VX_PF_GRAIN, up to
+ * VX_PF_ROWS); where the device has no room for them, or the attention keeps a
+ * partial per 32 positions (other head sizes), VX_PF_GRAIN rows. */
+static vx_error pf_alloc(vx_dev *d, int P)
+{
+    int R = (P + VX_PF_GRAIN - 1) / VX_PF_GRAIN * VX_PF_GRAIN;
+    const int most = d->hd == 64 || d->hd == 128 ? VX_PF_ROWS : VX_PF_GRAIN;
+    if (R > most) R = most;
+    if (d->pf_rows >= R) {
+        if (d->pf_ws_ctx == d->n_ctx_alloc && d->pf_ws_cap == d->opt.attn_cap) return VX_OK;
+        /* a cache allocated again for another n_ctx, or another cap: the
+         * attention workspace is sized for both */
+        TRY(vxh_stream_sync(d->stream));
+        vxh_workspace_free(&d->pf_ws);
+        d->pf_ws_ctx = -1;
+        return pf_ws_alloc(d, d->pf_rows);
+    }
+    if (d->pf_rows) TRY(vxh_stream_sync(d->stream));
+    pf_free(d);
+    vx_error e = pf_alloc_rows(d, R);
+    if (e != VX_OK && R > VX_PF_GRAIN) {
+        pf_free(d);
+        e = pf_alloc_rows(d, VX_PF_GRAIN);
+    }
+    if (e != VX_OK) pf_free(d);
+    return e;
+}
+
+/* M <= pf_rows prompt rows at positions n_past .. n_past+M-1 (all below
  * n_ctx) as one batch: per layer RMSNorm rows, the large-M GEMMs, RoPE + KV
  * store, causal attention over the cache, SwiGLU (src/model.c:514-594).
  * With last_logits the last row's logits land in d->logits row 0. */
@@ -1195,8 +1226,7 @@ static vx_error forward_prefill(vx_model *m, const int *tokens, int M, int n_pas
     vx_dev *d = vx_dev_of(m);
     const int dd = d->d, kvd = d->kvd, n_ctx = d->n_ctx_alloc;
     vxh_stream s = d->stream;
-    vx_error e = pf_alloc(d);
-    if (e != VX_OK) return e;
+    vx_error e;
     TRY(vxh_upload(d->pf_tok, tokens, sizeof(int) * (size_t)M, s));
     if (d->has_embd) TRY(vxh_qmat_gather_rows(&d->embd, d->pf_tok, M, vx_get_synthetic_weight_scale(), d->pf_x, dd, s));
     else TRY(vxh_fill_f32(d->pf_x, 0.0f, (size_t)M * dd, s));
@@ -1209,8 +1239,8 @@ static vx_error forward_prefill(vx_model *m, const int *tokens, int M, int n_pas
                           scale_for(d, Ld->wqkv.type), s));
         TRY(vxh_rope_kv_rows(d->pf_qkv, d->ld_qkv, M, n_past, n_ctx, d->n_heads, d->n_kv, d->hd, Ld->bq, Ld->bk,
                              Ld->bv, d->rope_cos, d->rope_sin, d->n_pos, d->pf_q, dd, kc, vc, s));
-        TRY(vxh_attention(d->pf_q, M, n_past, n_ctx, d->n_heads, d->n_kv, d->hd, d->opt.attn_cap, kc, vc,
-                          d->pf_att, dd, &d->pf_ws, s));
+        TRY(vxh_attention_rows(d->pf_q, M, n_past, n_ctx, d->n_heads, d->n_kv, d->hd, d->opt.attn_cap, kc, vc,
+                               d->pf_att, dd, &d->pf_ws, s));
         if (Ld->has_o) {
             TRY(vxh_rows_panel(d->pf_att, dd, M, dd, d->pf_px, s));
             TRY(vxh_gemm_rows(&Ld->wo, d->pf_px, M, d->pf_x, dd, dd, d->pf_x, dd, scale_for(d, Ld->wo.type), s));
@@ -1268,6 +1298,8 @@ vx_error vx_dev_run_tokens(vx_model *m, const int *tokens, int n, int logits_mod
             if (P > VX_PF_ROWS) P = VX_PF_ROWS;
             if (P > n_ctx - c) P = n_ctx - c;
             if (P >= d->opt.prefill_min_rows) {
+                if ((e = pf_alloc(d, P)) != VX_OK) return e;
+                if (P > d->pf_rows) P = d->pf_rows;
                 const int last = i + P == n && logits_mode == VX_LOGITS_LAST;
                 if ((e = forward_prefill(m, tokens + i, P, c, last)) != VX_OK) return e;
                 if (last) TRY(vxh_download(logits_host, d->logits, sizeof(float) * (size_t)V, d->stream));

@@ -14,7 +14,11 @@
 #include "vxh.h"
 
 #define VX_MAX_BATCH 16
-#define VX_PF_ROWS 512             /* rows of one large-M prefill chunk */
+/* rows of one large-M prefill chunk: 2048 x 4096-column matrices fill the GEMM
+ * with whole-K workgroups (four 512-row chunks of a 7B-shape layer take 2.21 ms
+ * in its GEMMs, one of 2048 rows 1.77) */
+#define VX_PF_ROWS 2048
+#define VX_PF_GRAIN 512            /* its buffers grow in steps of this many rows */
 
 /* ---- errors ----------------------------------------------------------------- */
 void vx_set_error(const char *fmt, ...);
@@ -109,9 +113,9 @@ typedef struct vx_dev {
     double *acc_y;
     /* large-M prompt prefill (allocated on first use): token ids, the
      * residual rows, normed rows, q|k|v rows, rotated q, attention rows,
-     * gate/up rows, SwiGLU rows, each [VX_PF_ROWS][...] fp32, and the
+     * gate/up rows, SwiGLU rows, each [pf_rows][...] fp32, and the
      * attention workspace for that many rows */
-    int pf_ready;
+    int pf_rows;                       /* rows the buffers hold (0: not allocated) */
     int pf_ws_ctx, pf_ws_cap;          /* n_ctx_alloc and attn_cap pf_ws was sized for */
     int *pf_tok;
     float *pf_x, *pf_xn, *pf_qkv, *pf_q, *pf_att, *pf_gu, *pf_h;
