@@ -1140,6 +1140,43 @@ __global__ __launch_bounds__(CMB_THREADS) void vx_attention_combine_kernel(
     }
 }
 
+// The prompt kernel's few segments joined: HD/4 threads per query, every
+// segment's (max, sum, acc) read once, no exchange between threads.  Bound by
+// reading the partials: 2048 x 32 heads of 128, two segments: 66 -> 20 us with
+// the kernel above, which puts 256 threads and two barriers on each query.
+template <int HD>
+__global__ __launch_bounds__(256) void vx_attention_join_kernel(const float *__restrict__ part, int M, int n_heads,
+                                                                int n_kv, int n_seg, float *__restrict__ out,
+                                                                int ld_out)
+{
+    constexpr int L4 = HD / 4;
+    const int G = n_heads / n_kv, QM = G * M;
+    const long i = (long)blockIdx.x * (256 / L4) + threadIdx.x / L4;    // query: (kv head, hl, row)
+    if (i >= (long)n_kv * QM) return;
+    const int d4 = threadIdx.x % L4, g = (int)(i / QM), qi = (int)(i % QM), m = qi % M, head = g * G + qi / M;
+    const size_t cstride = (size_t)QM * PART_STRIDE(HD);
+    const float *pq = part + (size_t)g * n_seg * cstride + (size_t)qi * PART_STRIDE(HD);
+    float mx = -INFINITY;
+    for (int c = 0; c < n_seg; c++) mx = fmaxf(mx, pq[c * cstride]);
+    float l = 0.0f;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int c = 0; c < n_seg; c++) {
+        const float *pc = pq + c * cstride;
+        const float cm = pc[0];
+        if (cm == -INFINITY) continue;       // a segment past the query's positions: sums not written
+        const float f = expf(cm - mx);
+        const float4 v = *(const float4 *)(pc + 4 + 4 * d4);
+        l = fmaf(f, pc[1], l);
+        a.x = fmaf(f, v.x, a.x);
+        a.y = fmaf(f, v.y, a.y);
+        a.z = fmaf(f, v.z, a.z);
+        a.w = fmaf(f, v.w, a.w);
+    }
+    const float inv = 1.0f / (l + 1e-10f);
+    *(float4 *)(out + (size_t)m * ld_out + (size_t)head * HD + 4 * d4) =
+        make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+}
+
 // LDS of a workgroup holding nq queries; the query split keeps it <= 64 KiB.
 static size_t vx_attn_lds(int nq, int hd)
 {
@@ -1185,6 +1222,9 @@ static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int *seg_t)
     *seg_t = (n_t + n_seg - 1) / n_seg;
     return (n_t + *seg_t - 1) / *seg_t;
 }
+
+// up to this many segments are joined by one thread per four outputs, in turn
+#define VX_JOIN_SEGMENTS 32
 
 // What any batch of up to M rows over up to ctx positions needs: the chunk
 // kernels' partials where they run (VX_ATT_MFMA_MAX_M rows, or fewer scores
@@ -1304,6 +1344,17 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
                                                                       nqg, n_seg, seg_t * AR_T, ws->part, out, ld_out);
         VXH_LAUNCHED();
         if (n_seg == 1) return VXH_OK;
+        if (n_seg <= VX_JOIN_SEGMENTS) {
+            const unsigned jg = (unsigned)(((long)n_kv_heads * QM * (head_dim / 4) + 255) / 256);
+            if (head_dim == 64)
+                vx_attention_join_kernel<64><<<jg, 256, 0, vxh_hs(s)>>>(ws->part, M, n_heads, n_kv_heads, n_seg, out,
+                                                                        ld_out);
+            else
+                vx_attention_join_kernel<128><<<jg, 256, 0, vxh_hs(s)>>>(ws->part, M, n_heads, n_kv_heads, n_seg, out,
+                                                                         ld_out);
+            VXH_LAUNCHED();
+            return VXH_OK;
+        }
         return vx_attention_combine(ws->part, M, n_heads, n_kv_heads, head_dim, n_seg, out, ld_out, nullptr, 0, s);
     }
     size_t lds = vx_attn_lds(qpg, head_dim);
