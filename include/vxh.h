@@ -355,12 +355,18 @@ int vxh_acc_store_norm(double *acc, int ld_acc, int M, int n, float *y, int ldy,
  *
  * vxh_gemm_rows: Y[m][n] = (R ? R[m][n] : 0) + scale * sum_k X[m][k] W[n][k]
  * for m < M (any M >= 1), n < n_out, from the rows panel of X (built with
- * K = W->n_cols).  Compute-bound MFMA tiles of 64 rows x 128 columns;
- * weights enter as the exact fp16 pair d*q = hi + lo and the activations as
- * fp16 hi + lo, summed over all of K in fp32 (within the fp32 GEMV's
- * rounding of src/quantize.c:728-750).  Y may alias R. */
+ * K = W->n_cols).  Compute-bound MFMA tiles of 64 rows; a block's whole
+ * numbers times the activations' fp16 hi and lo parts, scaled by the block's
+ * d and summed in fp32 (within the fp32 GEMV's rounding of
+ * src/quantize.c:728-750).  Y may alias R.
+ *
+ * vxh_rmsnorm_rows_panel / vxh_swiglu_rows_panel: the panel of vxh_rmsnorm of
+ * X (w may be NULL; 16-byte aligned), and of vxh_swiglu_rows of gu (F % 32 ==
+ * 0, ld_gu % 4 == 0), without the fp32 rows in between. */
 size_t vxh_rows_panel_bytes(int M, int K);
 int vxh_rows_panel(const float *X, int ldx, int M, int K, void *px, vxh_stream s);
+int vxh_rmsnorm_rows_panel(const float *X, int ldx, int M, int K, const float *w, void *px, vxh_stream s);
+int vxh_swiglu_rows_panel(const float *gu, int ld_gu, int M, int F, float thr, void *px, vxh_stream s);
 int vxh_gemm_rows(const vxh_qmat *W, const void *px, int M, float *Y, int ldy, int n_out,
                   const float *R, int ldr, float scale, vxh_stream s);
 /* vxh_rope_kv for fp32 q|k|v rows qkv[M][ld_qkv] (no deferred norm, not

@@ -245,6 +245,66 @@ def test_rows_gemm_row_scales(P, typ, mag):
     assert ok, max_violation(g, o)
 
 
+@pytest.mark.parametrize("M,K", [(1, 32), (7, 1056), (64, 4096), (65, 96), (100, 11264), (9, 11296), (33, 22560),
+                                 (1024, 96), (1030, 4096), (1025, 4128), (1024, 11296)])
+@pytest.mark.parametrize("kind", ["rmsnorm", "rmsnorm_w", "swiglu"])
+def test_rows_panel_kinds(P, kind, M, K):
+    """The fused panels against the panel of the same rows from vxh_rmsnorm /
+    vxh_swiglu_rows (rows in registers and longer ones, ragged row groups, odd
+    block counts).  The swiglu rows are the same floats, so the panels are the
+    same bytes; the norm's sum of squares may be added in another order,
+    which moves 1/rms by a few of its roundings (2^-20 allowed), and the two
+    fp16 parts keep 2^-21 of the row's largest."""
+    print(f"rows panel {kind} M={M} K={K}", flush=True)
+    vp = C.c_void_p
+    L = N.bind_vxh(P)
+    f, i = C.c_float, C.c_int
+    L.vxh_rows_panel_bytes.restype, L.vxh_rows_panel_bytes.argtypes = C.c_size_t, [i, i]
+    L.vxh_rows_panel.argtypes = [vp, i, i, i, vp, vp]
+    L.vxh_rmsnorm.argtypes = [vp, i, i, i, vp, vp, i, vp]
+    L.vxh_swiglu_rows.argtypes = [vp, i, i, i, f, vp, i, vp]
+    L.vxh_rmsnorm_rows_panel.argtypes = [vp, i, i, i, vp, vp, vp]
+    L.vxh_swiglu_rows_panel.argtypes = [vp, i, i, i, f, vp, vp]
+    rng = np.random.default_rng(M + K)
+    ld = 2 * K if kind == "swiglu" else K + 4
+    x = (rng.normal(0, 1, (M, ld)) * np.exp(rng.normal(0, 3, (M, 1)))).astype(np.float32)
+    w = rng.normal(1, 0.2, K).astype(np.float32)
+    dx, dw, dh = N.DevBuf(L, x), N.DevBuf(L, w), N.DevBuf(L, nbytes=4 * M * K)
+    nb = L.vxh_rows_panel_bytes(M, K)
+    pa, pb = (N.DevBuf(L, np.zeros(nb, np.uint8)) for _ in range(2))
+    wp = dw.ptr if kind == "rmsnorm_w" else None
+    if kind == "swiglu":
+        assert L.vxh_swiglu_rows(dx.ptr, ld, M, K, 0.01, dh.ptr, K, None) == 0
+        assert L.vxh_swiglu_rows_panel(dx.ptr, ld, M, K, 0.01, pb.ptr, None) == 0
+    else:
+        assert L.vxh_rmsnorm(dx.ptr, ld, M, K, wp, dh.ptr, K, None) == 0
+        assert L.vxh_rmsnorm_rows_panel(dx.ptr, ld, M, K, wp, pb.ptr, None) == 0
+    assert L.vxh_rows_panel(dh.ptr, K, M, K, pa.ptr, None) == 0
+    assert L.vxh_stream_sync(None) == 0
+    a, b = pa.get(np.uint8, nb), pb.get(np.uint8, nb)
+    rows, n_pairs = (M + 63) // 64 * 64, (K + 63) // 64
+
+    def decode(p):
+        """[row][column] of a panel, row scales applied."""
+        s = p[:rows * n_pairs * 256].view(np.float16).astype(np.float64)
+        s = s.reshape(rows // 64, n_pairs, 2, 2, 2, 2, 2, 32, 8)   # rg, pair, mt, blk, s, hi/lo, half, row, element
+        v = s.sum(axis=5).transpose(0, 2, 6, 1, 3, 5, 4, 7)        # rg, mt, row, pair, blk, half, s, element
+        v = v.reshape(rows, n_pairs * 64)
+        rs = p[rows * n_pairs * 256:][:4 * M].view(np.float32).astype(np.float64)
+        return v[:M] * rs[:, None], v[M:]
+
+    (va, ta), (vb, tb) = decode(a), decode(b)
+    h = dh.get(np.float32, M * K).reshape(M, K).astype(np.float64)
+    assert not ta.any() and not tb.any() and not vb[:, K:].any()
+    assert np.all(np.abs(va[:, :K] - h) <= 2.0 ** -22 * np.abs(h).max(axis=1, keepdims=True))
+    if kind == "swiglu":
+        assert np.array_equal(a, b)
+    else:
+        assert np.all(np.abs(vb[:, :K] - h) <= 2.0 ** -20 * np.abs(h) + 2.0 ** -21 * np.abs(h).max(axis=1, keepdims=True))
+    for buf in (dx, dw, dh, pa, pb):
+        buf.free()
+
+
 @pytest.mark.parametrize("typ", [GGML_Q4_0, GGML_Q8_0])
 @pytest.mark.parametrize("M,rows,cols", [
     (1, 1, 32), (17, 300, 128), (32, 96, 544), (33, 33, 1120), (65, 4096, 96), (96, 2080, 544),

@@ -313,55 +313,154 @@ static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
     return vx_pf_gemm_launch<QT, 1, 1, 8>(a, s);
 }
 
-// Rows panel: fp32 rows x[M][ldx] as the GEMM's LDS stages.  Unit u of a
-// (row group rg, pair p) stage, u = ((mt*2 + blk)*2 + s)*64 + ln, holds row
-// 64 rg + 32 mt + ln % 32, elements 64 p + 32 blk + 16 (ln/32) + 8 s .. + 7,
-// as hi = fp16(x') and (64 units further) lo = fp16(x' - hi).  One workgroup
-// per row: x' = x 2^-e with e from the row's largest magnitude (vx_row_scale:
-// |x'| < 1), so no element overflows fp16 and a row of small values keeps
-// the low parts' bits; rs[row] = 2^e goes back in in the GEMM epilogue,
-// exactly.  Rows past M (up to the 64-row group) and columns past K are
-// zeros.
-__global__ __launch_bounds__(256) void vx_pf_panel_kernel(const float *__restrict__ x, int ldx, int M, int K,
-                                                          int n_pairs, uint4 *__restrict__ px, float *__restrict__ rs)
+// Rows panel: fp32 rows as the GEMM's LDS stages.  Unit u of a (row group
+// rg, pair p) stage, u = ((mt*2 + blk)*2 + s)*128 + ln, holds row 64 rg + 32 mt
+// + ln % 32, elements 64 p + 32 blk + 16 (ln/32) + 8 s .. + 7, as hi = fp16(x')
+// and (64 units further) lo = fp16(x' - hi).  x' = x 2^-e with e from the row's
+// largest magnitude (vx_row_scale: |x'| < 1), so no element overflows fp16 and
+// a row of small values keeps the low parts' bits; rs[row] = 2^e goes back in
+// in the GEMM epilogue, exactly.  Rows past M (up to the 64-row group) and
+// columns past K are zeros.
+//
+// The rows are x[M][ldx] as they are (PF_ROWS), their RMSNorm (PF_RMS), or the
+// SwiGLU with the FFN gate-skip (src/model.c:582-585) of the interleaved
+// gate/up product (PF_SWIGLU; 16 gate then 16 up columns per tile of 32).
+//
+// Bound by memory.  A workgroup takes PR rows, WPR wavefronts each.  Many
+// rows: 8 and 2, as the 16-byte units of 8 rows are one 128-byte line; with a
+// workgroup per row the rows of a line go to 8 XCDs, whose L2s each write back
+// a part of it (2048 x 4096: 33 -> 19 us; norm and panel 50 -> 21; SwiGLU and
+// panel of 2048 x 11008 155 -> 62).  Few rows: a workgroup each (77 x 11008
+// 7.4 us, 22 with 8 rows: only 16 workgroups).  A row stays in registers, up
+// to KEEP groups of 8 columns per lane; what is left is read again.
+enum { PF_ROWS = 0, PF_RMS = 1, PF_SWIGLU = 2 };
+
+template <int SRC, int KEEP, int PR, int WPR>
+__global__ __launch_bounds__(64 * PR *WPR) void vx_pf_panel_kernel(const float *__restrict__ x, int ldx, int M, int K,
+                                                                    int n_pairs, const float *__restrict__ w, float thr,
+                                                                    uint4 *__restrict__ px, float *__restrict__ rs)
 {
-    const int row = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = wave % PR, part = wave / PR;
+    const int row = blockIdx.x * PR + r;
     const int rg = row / PF_BM, mt = (row % PF_BM) / 32, l32 = row % 32;
     const bool live = row < M;
     const float *xr = x + (size_t)(live ? row : 0) * ldx;
-    __shared__ float red[4];
-    float amax = 0.0f;
-    if (live)
-        for (int k = 8 * threadIdx.x; k < K; k += 8 * 256) {
-            const float4 a = *(const float4 *)(xr + k), b = *(const float4 *)(xr + k + 4);
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w))));
+    __shared__ float red[2][WPR][PR];
+    const int k0 = 8 * (lane + 64 * part), step = 8 * 64 * WPR;
+    // the 8 columns from k on, before any norm; zeros past K and M (K % 32 ==
+    // 0: wholly in or out), read from a clamped address so that the loads of
+    // all groups leave together
+    auto load = [&](int k, float v[8]) {
+        const bool ok = live && k < K;
+        const int kc = min(k, K - 8);
+        const float *p = SRC == PF_SWIGLU ? xr + 32 * (kc / 16) + kc % 16 : xr + kc;
+        const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
+        const float t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        if constexpr (SRC == PF_SWIGLU) {
+            const float4 ua = *(const float4 *)(p + 16), ub = *(const float4 *)(p + 20);
+            const float u[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float g = vx_silu(t[e]);
+                v[e] = !ok || fabsf(g) < thr ? 0.0f : g * u[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = ok ? t[e] : 0.0f;
         }
-    amax = vx_wave_max64(amax);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    };
+    // the norm's weights of the same columns (1 without them)
+    auto load_w = [&](int k, float wv[8]) {
+        float4 a = make_float4(1.f, 1.f, 1.f, 1.f), b = a;
+        if (w) {
+            const float *p = w + min(k, K - 8);
+            a = *(const float4 *)p;
+            b = *(const float4 *)(p + 4);
+        }
+        wv[0] = a.x; wv[1] = a.y; wv[2] = a.z; wv[3] = a.w;
+        wv[4] = b.x; wv[5] = b.y; wv[6] = b.z; wv[7] = b.w;
+    };
+    float inv = 1.0f;
+    auto norm = [&](const float wv[8], float v[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = wv[e] * (v[e] * inv);
+    };
+    auto load_normed = [&](int k, float v[8]) {
+        load(k, v);
+        if constexpr (SRC == PF_RMS) {
+            float wv[8];
+            load_w(k, wv);
+            norm(wv, v);
+        }
+    };
+    // the values of a row's wavefronts joined
+    auto join = [&](int slot, float v, bool sum) {
+        if (lane == 0) red[slot][part][r] = v;
+        __syncthreads();
+        float j = red[slot][0][r];
+#pragma unroll
+        for (int i = 1; i < WPR; i++) j = sum ? j + red[slot][i][r] : fmaxf(j, red[slot][i][r]);
+        return j;
+    };
+    float keep[KEEP][8];
+    float wk[SRC == PF_RMS ? KEEP : 1][8];
+#pragma unroll
+    for (int i = 0; i < KEEP; i++) {
+        load(k0 + i * step, keep[i]);
+        if constexpr (SRC == PF_RMS) load_w(k0 + i * step, wk[i]);
+    }
+    if constexpr (SRC == PF_RMS) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < KEEP; i++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) ss += keep[i][e] * keep[i][e];
+        for (int k = k0 + KEEP * step; k < K; k += step) {
+            float v[8];
+            load(k, v);
+#pragma unroll
+            for (int e = 0; e < 8; e++) ss += v[e] * v[e];
+        }
+        inv = vx_rms_inv(join(0, vx_wave_sum64(ss), true), K);
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < KEEP; i++) {
+        if constexpr (SRC == PF_RMS) norm(wk[i], keep[i]);
+#pragma unroll
+        for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(keep[i][e]));
+    }
+    for (int k = k0 + KEEP * step; k < K; k += step) {
+        float v[8];
+        load_normed(k, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+    }
+    amax = join(1, vx_wave_max64(amax), false);
     float rsv;
     const float sc = live ? vx_row_scale(amax, &rsv) : 1.0f;
-    if (live && threadIdx.x == 0) rs[row] = rsv;
-    for (int k = 8 * threadIdx.x; k < n_pairs * 64; k += 8 * 256) {
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (live && k < K) {   // K % 32 == 0: a block is wholly in range or out
-            const float4 a = *(const float4 *)(xr + k), b = *(const float4 *)(xr + k + 4);
-            v[0] = a.x * sc; v[1] = a.y * sc; v[2] = a.z * sc; v[3] = a.w * sc;
-            v[4] = b.x * sc; v[5] = b.y * sc; v[6] = b.z * sc; v[7] = b.w * sc;
-        }
+    if (live && lane == 0 && part == 0) rs[row] = rsv;
+    auto put = [&](int k, const float v[8]) {
         vx_half8 hi, lo;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const _Float16 t = (_Float16)v[e];
-            hi[e] = t;
-            lo[e] = (_Float16)(v[e] - (float)t);
+            const float t = v[e] * sc;
+            const _Float16 f = (_Float16)t;
+            hi[e] = f;
+            lo[e] = (_Float16)(t - (float)f);
         }
         const int p = k / 64, blk = (k / 32) & 1, half = (k / 16) & 1, s = (k / 8) & 1;
         uint4 *o = px + ((size_t)rg * n_pairs + p) * PF_STAGE + ((mt * 2 + blk) * 2 + s) * 128 + l32 + 32 * half;
         o[0] = __builtin_bit_cast(uint4, hi);
         o[64] = __builtin_bit_cast(uint4, lo);
+    };
+#pragma unroll
+    for (int i = 0; i < KEEP; i++)
+        if (k0 + i * step < n_pairs * 64) put(k0 + i * step, keep[i]);
+    for (int k = k0 + KEEP * step; k < n_pairs * 64; k += step) {
+        float v[8];
+        load_normed(k, v);
+        put(k, v);
     }
 }
 
@@ -377,16 +476,49 @@ extern "C" size_t vxh_rows_panel_bytes(int M, int K)
     return vx_pf_stage_bytes(M, K) + ((size_t)M * sizeof(float) + 15) / 16 * 16;
 }
 
+// from here 8 rows to a workgroup (1024 x 4096: 17.3 us with one each, 12.2;
+// below, they would leave more than half of the CUs idle)
+#define PF_MANY_ROWS 1024
+
+template <int SRC>
+static int vx_pf_panel(const float *x, int ldx, int M, int K, const float *w, float thr, void *px, vxh_stream s)
+{
+    const int n_pairs = (K + 63) / 64;
+    const unsigned rows = (unsigned)((M + PF_BM - 1) / PF_BM * PF_BM);
+    float *rs = (float *)((char *)px + vx_pf_stage_bytes(M, K));
+    if (M < PF_MANY_ROWS)
+        vx_pf_panel_kernel<SRC, 6, 1, 4><<<rows, 256, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px, rs);
+    else if (K <= 4 * 1024)
+        vx_pf_panel_kernel<SRC, 4, 8, 2><<<rows / 8, 1024, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px,
+                                                                         rs);
+    else
+        vx_pf_panel_kernel<SRC, SRC == PF_RMS ? 6 : 11, 8, 2><<<rows / 8, 1024, 0, vxh_hs(s)>>>(
+            x, ldx, M, K, n_pairs, w, thr, (uint4 *)px, rs);
+    VXH_LAUNCHED();
+    return VXH_OK;
+}
+
 extern "C" int vxh_rows_panel(const float *X, int ldx, int M, int K, void *px, vxh_stream s)
 {
     if (!X || !px || M < 1 || K < 32 || K % 32 || ldx < K || ldx % 4 || ((uintptr_t)X & 15) || ((uintptr_t)px & 15))
         return vxh_fail(VXH_ERR_PARAM, "rows_panel: M %d K %d ldx %d", M, K, ldx);
-    const int n_pairs = (K + 63) / 64;
-    const unsigned rows = (unsigned)((M + PF_BM - 1) / PF_BM * PF_BM);
-    vx_pf_panel_kernel<<<rows, 256, 0, vxh_hs(s)>>>(X, ldx, M, K, n_pairs, (uint4 *)px,
-                                                     (float *)((char *)px + vx_pf_stage_bytes(M, K)));
-    VXH_LAUNCHED();
-    return VXH_OK;
+    return vx_pf_panel<PF_ROWS>(X, ldx, M, K, nullptr, 0.0f, px, s);
+}
+
+extern "C" int vxh_rmsnorm_rows_panel(const float *X, int ldx, int M, int K, const float *w, void *px, vxh_stream s)
+{
+    if (!X || !px || M < 1 || K < 32 || K % 32 || ldx < K || ldx % 4 || ((uintptr_t)X & 15) || ((uintptr_t)px & 15) ||
+        ((uintptr_t)w & 15))
+        return vxh_fail(VXH_ERR_PARAM, "rmsnorm_rows_panel: M %d K %d ldx %d", M, K, ldx);
+    return vx_pf_panel<PF_RMS>(X, ldx, M, K, w, 0.0f, px, s);
+}
+
+extern "C" int vxh_swiglu_rows_panel(const float *gu, int ld_gu, int M, int F, float thr, void *px, vxh_stream s)
+{
+    if (!gu || !px || M < 1 || F < 32 || F % 32 || ld_gu < 2 * F || ld_gu % 4 || ((uintptr_t)gu & 15) ||
+        ((uintptr_t)px & 15))
+        return vxh_fail(VXH_ERR_PARAM, "swiglu_rows_panel: M %d F %d ld %d", M, F, ld_gu);
+    return vx_pf_panel<PF_SWIGLU>(gu, ld_gu, M, F, nullptr, thr, px, s);
 }
 
 extern "C" int vxh_gemm_rows(const vxh_qmat *W, const void *px, int M, float *Y, int ldy, int n_out,

@@ -160,10 +160,10 @@ static void prof_free(vx_dev *d);
 
 static void pf_free(vx_dev *d)
 {
-    vxh_free(d->pf_tok); vxh_free(d->pf_x); vxh_free(d->pf_xn); vxh_free(d->pf_qkv);
-    vxh_free(d->pf_q); vxh_free(d->pf_att); vxh_free(d->pf_gu); vxh_free(d->pf_h); vxh_free(d->pf_px);
+    vxh_free(d->pf_tok); vxh_free(d->pf_x); vxh_free(d->pf_qkv);
+    vxh_free(d->pf_q); vxh_free(d->pf_att); vxh_free(d->pf_gu); vxh_free(d->pf_px);
     d->pf_tok = NULL;
-    d->pf_x = d->pf_xn = d->pf_qkv = d->pf_q = d->pf_att = d->pf_gu = d->pf_h = NULL;
+    d->pf_x = d->pf_qkv = d->pf_q = d->pf_att = d->pf_gu = NULL;
     d->pf_px = NULL;
     vxh_workspace_free(&d->pf_ws);
     d->pf_rows = 0;
@@ -1177,12 +1177,10 @@ static vx_error pf_alloc_rows(vx_dev *d, int rows)
     const size_t R = rows;
     TRY(vxh_malloc((void **)&d->pf_tok, sizeof(int) * R));
     TRY(vxh_malloc((void **)&d->pf_x, sizeof(float) * R * d->d));
-    TRY(vxh_malloc((void **)&d->pf_xn, sizeof(float) * R * d->d));
     TRY(vxh_malloc((void **)&d->pf_qkv, sizeof(float) * R * d->ld_qkv));
     TRY(vxh_malloc((void **)&d->pf_q, sizeof(float) * R * d->d));
     TRY(vxh_malloc((void **)&d->pf_att, sizeof(float) * R * d->d));
     TRY(vxh_malloc((void **)&d->pf_gu, sizeof(float) * R * d->ld_gu));
-    TRY(vxh_malloc((void **)&d->pf_h, sizeof(float) * R * d->F));
     TRY(vxh_malloc(&d->pf_px, vxh_rows_panel_bytes(rows, d->F > d->d ? d->F : d->d)));
     vx_error e = pf_ws_alloc(d, rows);
     if (e == VX_OK) d->pf_rows = rows;
@@ -1233,8 +1231,7 @@ static vx_error forward_prefill(vx_model *m, const int *tokens, int M, int n_pas
     for (int l = 0; l < d->n_layers; l++) {
         vx_dev_layer *Ld = &d->layers[l];
         float *kc = m->k_cache + (size_t)l * n_ctx * kvd, *vc = m->v_cache + (size_t)l * n_ctx * kvd;
-        TRY(vxh_rmsnorm(d->pf_x, dd, M, dd, Ld->attn_norm, d->pf_xn, dd, s));
-        TRY(vxh_rows_panel(d->pf_xn, dd, M, dd, d->pf_px, s));
+        TRY(vxh_rmsnorm_rows_panel(d->pf_x, dd, M, dd, Ld->attn_norm, d->pf_px, s));
         TRY(vxh_gemm_rows(&Ld->wqkv, d->pf_px, M, d->pf_qkv, d->ld_qkv, dd + 2 * kvd, NULL, 0,
                           scale_for(d, Ld->wqkv.type), s));
         TRY(vxh_rope_kv_rows(d->pf_qkv, d->ld_qkv, M, n_past, n_ctx, d->n_heads, d->n_kv, d->hd, Ld->bq, Ld->bk,
@@ -1246,12 +1243,10 @@ static vx_error forward_prefill(vx_model *m, const int *tokens, int M, int n_pas
             TRY(vxh_gemm_rows(&Ld->wo, d->pf_px, M, d->pf_x, dd, dd, d->pf_x, dd, scale_for(d, Ld->wo.type), s));
         } else
             TRY(vxh_add_rows(d->pf_x, dd, d->pf_att, dd, M, dd, s));
-        TRY(vxh_rmsnorm(d->pf_x, dd, M, dd, Ld->ffn_norm, d->pf_xn, dd, s));
-        TRY(vxh_rows_panel(d->pf_xn, dd, M, dd, d->pf_px, s));
+        TRY(vxh_rmsnorm_rows_panel(d->pf_x, dd, M, dd, Ld->ffn_norm, d->pf_px, s));
         TRY(vxh_gemm_rows(&Ld->wgu, d->pf_px, M, d->pf_gu, d->ld_gu, d->ld_gu, NULL, 0,
                           scale_for(d, Ld->wgu.type), s));
-        TRY(vxh_swiglu_rows(d->pf_gu, d->ld_gu, M, d->F, d->opt.ffn_gate_threshold, d->pf_h, d->F, s));
-        TRY(vxh_rows_panel(d->pf_h, d->F, M, d->F, d->pf_px, s));
+        TRY(vxh_swiglu_rows_panel(d->pf_gu, d->ld_gu, M, d->F, d->opt.ffn_gate_threshold, d->pf_px, s));
         TRY(vxh_gemm_rows(&Ld->wd, d->pf_px, M, d->pf_x, dd, dd, d->pf_x, dd, scale_for(d, Ld->wd.type), s));
     }
     if (!last_logits) return VX_OK;

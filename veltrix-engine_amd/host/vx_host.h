@@ -112,13 +112,13 @@ typedef struct vx_dev {
     float *x2;
     double *acc_y;
     /* large-M prompt prefill (allocated on first use): token ids, the
-     * residual rows, normed rows, q|k|v rows, rotated q, attention rows,
-     * gate/up rows, SwiGLU rows, each [pf_rows][...] fp32, and the
-     * attention workspace for that many rows */
+     * residual rows, q|k|v rows, rotated q, attention rows, gate/up rows,
+     * each [pf_rows][...] fp32, and the attention workspace for that many
+     * rows */
     int pf_rows;                       /* rows the buffers hold (0: not allocated) */
     int pf_ws_ctx, pf_ws_cap;          /* n_ctx_alloc and attn_cap pf_ws was sized for */
     int *pf_tok;
-    float *pf_x, *pf_xn, *pf_qkv, *pf_q, *pf_att, *pf_gu, *pf_h;
+    float *pf_x, *pf_qkv, *pf_q, *pf_att, *pf_gu;
     void *pf_px;                       /* rows panel of the GEMM input (vxh_rows_panel) */
     vxh_workspace pf_ws;
     /* GEMM profiling (vx_model_set_profiling) */
