@@ -281,6 +281,70 @@ def test_many_workgroup_kernels_equal_one_workgroup_kernels(P, V):
         b.free()
 
 
+@pytest.mark.parametrize("V", [1023, 1025, 65536, 65537, 131073, 196609, 262144, 262145])
+def test_many_workgroup_chunk_sizes(P, V):
+    """Either side of every chunk size (4 to 16 entries per thread, and rows
+    whose chunks are walked): row statistics against float64 (the sum of V
+    fp32 terms in chunks: 1e-5), the draw and a decision over two drafts
+    against the one-workgroup kernels (the same token unless the threshold
+    lies on a boundary within rounding)."""
+    print(f"chunk sizes V={V}", flush=True)
+    rng = np.random.default_rng(V)
+    ws = C.byref(vocab_ws(P))
+    T, k = 0.9, 2
+    Lg = rng.normal(0, 2.0, (k + 1, V)).astype(np.float32)
+    Lg[1, V - 1] = Lg[1].max() + 1.0  # the maximum in the last entry
+    D = (Lg[:k] + rng.normal(0, 0.5, (k, V))).astype(np.float32)
+    dL, dD = N.DevBuf(P, Lg), N.DevBuf(P, D)
+    ds, dn, dd = N.DevBuf(P, nbytes=4 * 3 * (k + 1)), N.DevBuf(P, nbytes=4 * 8 * k), N.DevBuf(P, nbytes=4 * k)
+    assert P.vxh_row_stats_mc(dL.ptr, V, k + 1, V, T, ds.ptr, ws, None) == 0, P.vxh_last_error()
+    st = ds.get(np.float32, 3 * (k + 1)).reshape(k + 1, 3)
+    assert np.array_equal(st[:, 0], Lg.max(axis=1))
+    assert np.array_equal(st[:, 2].view(np.int32), Lg.argmax(axis=1))
+    z = np.exp((Lg.astype(np.float64) - Lg.max(axis=1, keepdims=True)) / T)
+    assert np.allclose(st[:, 1], z.sum(axis=1), rtol=1e-5, atol=0)
+    ties = 0
+    for trial in range(12):
+        u = (rng.integers(0, 1 << 24, 2 * k + 1) / float(1 << 24)).astype(np.float32)
+        drafts = np.zeros(k, np.int32)
+        for i in range(k):
+            t1, n1 = sample_gpu(P, D[i], T, 1.0, u[i])
+            t2, n2 = sample_gpu(P, D[i], T, 1.0, u[i], True)
+            if t1 != t2:
+                p = np.exp((D[i].astype(np.float64) - D[i].max()) / T)
+                assert near_boundary(p / p.sum(), float(u[i])), (trial, i, t1, t2)
+                ties += 1
+            drafts[i] = t2
+            P.vxh_upload(C.c_void_p(dn.ptr.value + 32 * i), n2.ctypes.data_as(C.c_void_p), 32, None)
+        P.vxh_upload(dd.ptr, drafts.ctypes.data_as(C.c_void_p), 4 * k, None)
+        du = N.DevBuf(P, u[k:])
+        outs = []
+        for mc in (False, True):
+            out = N.DevBuf(P, np.full(k + 3, -1, np.int32))
+            if mc:
+                rc = P.vxh_accept_mc(dL.ptr, V, V, ds.ptr, dD.ptr, V, V, dn.ptr, dd.ptr, k, T, du.ptr, out.ptr, ws, None)
+            else:
+                rc = P.vxh_accept(dL.ptr, V, V, ds.ptr, dD.ptr, V, V, dn.ptr, dd.ptr, k, T, du.ptr, out.ptr, None)
+            assert rc == 0, P.vxh_last_error()
+            o = out.get(np.int32, k + 3)
+            outs.append(o[:2 + o[0]])
+            out.free()
+        du.free()
+        a, b = outs
+        assert np.array_equal(a[:-1], b[:-1]), (trial, a, b)
+        if a[-1] != b[-1]:
+            j = int(a[1])
+            w = z[j] / z[j].sum()
+            if j < k:
+                q = np.exp((D[j].astype(np.float64) - D[j].max()) / T)
+                w = np.maximum(0, w - q / q.sum())
+            assert near_boundary(w, float(u[2 * k])), (trial, a, b)
+            ties += 1
+    assert ties <= 1
+    for buf in (dL, dD, ds, dn, dd):
+        buf.free()
+
+
 def test_argmax_of_rows_without_a_maximum_is_index_zero(P):
     """A row with no value above -inf (all NaN, all -inf) has no first max;
     the kernels return index 0 (the reference's scan stays on its first
