@@ -449,6 +449,20 @@ def test_attention_qkv_matches_rope_then_attention(P, H, KV, hd, M, n_past, n_ct
         b.free()
 
 
+@pytest.mark.parametrize("H,KV,hd,M,n_past,n_ctx,cap", [
+    (28, 4, 128, 9, 4090, 4160, 0),       # four chunks per wavefront, new rows on both sides of a 256 edge
+    (28, 4, 128, 9, 4343, 4352, 0),       # the last row ends the cache and a 256-position workgroup
+    (28, 4, 128, 9, 8000, 8192, 4100),    # cap below the new rows: chunks that only store
+    (8, 8, 128, 1, 8200, 8192, 0),        # one row past the context, clamped to its last slot
+    (32, 4, 64, 9, 1015, 1100, 0),        # head_dim 64, two chunks: new rows across a 128 edge
+    (32, 32, 64, 16, 2032, 2048, 0),
+    (16, 8, 64, 9, 6135, 6200, 0)])       # head_dim 64, four chunks
+def test_attention_qkv_walks_several_chunks(P, H, KV, hd, M, n_past, n_ctx, cap):
+    """Enough positions for 2 and 4 chunks per wavefront, at their edges: the
+    output of the one-chunk kernel and the same cache rows."""
+    test_attention_qkv_matches_rope_then_attention(P, H, KV, hd, M, n_past, n_ctx, cap, True)
+
+
 def test_attention_qkv_rejects_clamped_batches(P):
     bind_attention(P)
     ws = Workspace()

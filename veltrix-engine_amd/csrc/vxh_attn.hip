@@ -263,7 +263,9 @@ __global__ __launch_bounds__(ATT_THREADS) void vx_attention_kernel(
 // 16 r (n = l % 16, r = l / 16):
 //  * QK^T, per 16 positions and per (j, i): A = K[position n][16 j + 4 r + i],
 //    B = q[query n][16 j + 4 r + i] (scaled by 1/sqrt(hd)); the result holds
-//    score(position 4 r + i, query n) in item i of lane (n, r).
+//    score(position 4 r + i, query n) in item i of lane (n, r).  Even and odd j
+//    sum in chains of their own: a third closer to the 64-bit result (4.2e-7 ->
+//    2.8e-7 at head_dim 128) at the same time.
 //  * P.V, per step s and chain c = 4 u + e: A = V[position 4 r + s][64 u +
 //    4 n + e], B = the probability in item s of lane (n, r); chain c
 //    accumulates output dim 64 u + 4 (4 r + i) + e of query n in item i.
@@ -659,18 +661,24 @@ __device__ __forceinline__ void vx_attention_mfma_body(
         vx_f32x4 S[NPG];
 #pragma unroll
         for (int pg = 0; pg < NPG; pg++) {
-            S[pg] = vx_f32x4{0.f, 0.f, 0.f, 0.f};
+            // two chains: no sum of products runs over more than half a head
+            vx_f32x4 S0 = {0.f, 0.f, 0.f, 0.f}, S1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                S[pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].x, qv[j].x, S[pg], 0, 0, 0);
-                S[pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].y, qv[j].y, S[pg], 0, 0, 0);
-                S[pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].z, qv[j].z, S[pg], 0, 0, 0);
-                S[pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].w, qv[j].w, S[pg], 0, 0, 0);
+            for (int j = 0; j < NJ; j += 2) {
+                S0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].x, qv[j].x, S0, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j + 1].x, qv[j + 1].x, S1, 0, 0, 0);
+                S0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].y, qv[j].y, S0, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j + 1].y, qv[j + 1].y, S1, 0, 0, 0);
+                S0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].z, qv[j].z, S0, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j + 1].z, qv[j + 1].z, S1, 0, 0, 0);
+                S0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j].w, qv[j].w, S0, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[pg][j + 1].w, qv[j + 1].w, S1, 0, 0, 0);
             }
 #pragma unroll
             for (int j = 0; j < NJ; j++)
-                asm volatile("" : "+v"(S[pg]) : "v"(__builtin_bit_cast(vx_f32x4, kr[pg][j])),
+                asm volatile("" : "+v"(S0), "+v"(S1) : "v"(__builtin_bit_cast(vx_f32x4, kr[pg][j])),
                              "v"(__builtin_bit_cast(vx_f32x4, qv[j])));
+            S[pg] = S0 + S1;
         }
         if (cc + 1 < NCW) load_k(tc + CH);        // the next chunk's K behind this chunk's V
         if constexpr (!V_EARLY) load_v(tc);
@@ -793,13 +801,7 @@ __device__ __forceinline__ void vx_attention_mfma_body(
 }
 
 // Work per wavefront of the fp32-MFMA kernels.
-// * NCW chunks per wavefront: the q-rows kernel at head_dim 128 (prompt
-//   prefill: many query groups per head, so half the wavefronts still fill the
-//   chip) walks two, V streaming behind K, and writes half the partials
-//   (rocprofv3, 2048-token prefill: 205 -> 188 us per launch).  At head_dim
-//   128 with q|k|v sums (the verify, nine rows) two chunks made the attention
-//   24 -> 27.6 us per layer: half as many wavefronts, each with a longer K -> V
-//   chain.
+// * NCW chunks per wavefront: 1 for q rows; vx_att_ncw for the q|k|v sums.
 // * NPG groups of 16 positions per chunk, MERGE: the draft decode (head_dim
 //   64, q|k|v sums, one row) has few wavefronts and each spends most of its
 //   time on its own instructions, so its wavefronts take 16 positions and the
@@ -807,13 +809,33 @@ __device__ __forceinline__ void vx_attention_mfma_body(
 //   positions for the output projection to combine).
 template <int HD, bool QKV>
 struct vx_att_cfg {
-    static constexpr int NCW = 1;
     static constexpr int NPG = QKV ? 1 : 2;
     static constexpr bool MERGE = QKV;
-    static constexpr int WCH = NCW * NPG * 16;
+    static constexpr int WCH = NPG * 16;
 };
+// 16-position chunks a wavefront of the q|k|v kernels walks, given the row
+// bytes of the cache and the wavefronts of one chunk each.  Walking several
+// derives the q vectors once for all of them, streams the next chunk's K behind
+// this one's V and leaves fewer partials, as long as enough wavefronts remain:
+// * head_dim 128: 4 once one-chunk wavefronts take more than a round (3072
+//   resident): 9 rows x 28/4 heads over 8192 positions 41.7 -> 29.2 us, over 4009
+//   22.9 -> 18.1; over 3009 (3024 wavefronts) 19.3 against 20.0.
+// * head_dim 64 (16 KB less per wavefront, more of them resident): 2 from 1200
+//   (9 x 32/4 over 1009: 12.2 -> 11.8), 4 from 6000 (16 x 14/2 over 8016: 22.8 ->
+//   18.3); at 4128 both 2 and 4 leave 9 x 32/32 over 2057 where it was.
+// * rows of 8 KB: as head_dim 64 from 3500 on (fp16, 9 x 32/32 x 128 over 2057:
+//   28.8, 27.7 with 2, 30.5 with 4; over 8009 68 -> 54 with 4).
+// * rows of 16 KB: always 1 (9 x 32/32 x 128 over 2057: 25.1, 27.6, 30.2 us; 2 rows
+//   over 8002: 57.6, 65.9, 65.8).
+static int vx_att_ncw(int head_dim, size_t row_bytes, long waves)
+{
+    if (row_bytes >= 16384) return 1;
+    const long two = head_dim == 64 ? 1200 : 3500, four = head_dim == 64 || row_bytes >= 8192 ? 6000 : 3500;
+    return waves >= four ? 4 : waves >= two ? 2 : 1;
+}
+
 // positions per wavefront and whether a workgroup merges its partials
-static void vx_att_geom(int head_dim, bool qkv, int *wch, bool *merge)
+static void vx_att_geom(int head_dim, bool qkv, int ncw, int *wch, bool *merge)
 {
     if (head_dim == 128) {
         *wch = qkv ? vx_att_cfg<128, true>::WCH : vx_att_cfg<128, false>::WCH;
@@ -822,6 +844,7 @@ static void vx_att_geom(int head_dim, bool qkv, int *wch, bool *merge)
         *wch = qkv ? vx_att_cfg<64, true>::WCH : vx_att_cfg<64, false>::WCH;
         *merge = qkv ? vx_att_cfg<64, true>::MERGE : vx_att_cfg<64, false>::MERGE;
     }
+    if (qkv) *wch *= ncw;
 }
 
 template <int HD, bool NT = false>
@@ -831,18 +854,20 @@ __global__ __launch_bounds__(ATT_THREADS) __attribute__((amdgpu_waves_per_eu(3))
     float *__restrict__ part, vx_qkv_args qa)
 {
     using C = vx_att_cfg<HD, false>;
-    vx_attention_mfma_body<false, HD, false, C::NCW, C::NPG, C::MERGE, NT>(
+    vx_attention_mfma_body<false, HD, false, 1, C::NPG, C::MERGE, NT>(
         q, M, n_past, n_ctx, n_heads, n_kv, cap, kc, vc, n_chunks, n_chunks_w, n_qg, part, qa);
 }
 
-template <int HD, bool KH = false, bool NT = false>
-__global__ __launch_bounds__(ATT_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void vx_attention_mfma_qkv_kernel(
+// two wavefronts per SIMD where head_dim 128 walks: K and V of a chunk live at
+// once spilled at three (9 rows x 28/4 heads over 8192 positions 32.0 -> 29.2 us)
+template <int HD, bool KH = false, bool NT = false, int NCW = 1>
+__global__ __launch_bounds__(ATT_THREADS) __attribute__((amdgpu_waves_per_eu(HD == 128 && NCW > 1 ? 2 : 3))) void vx_attention_mfma_qkv_kernel(
     const float *__restrict__ q, int M, int n_past, int n_ctx, int n_heads, int n_kv, int cap,
     float *__restrict__ kc, float *__restrict__ vc, int n_chunks, int n_chunks_w, int n_qg,
     float *__restrict__ part, vx_qkv_args qa)
 {
     using C = vx_att_cfg<HD, true>;
-    vx_attention_mfma_body<true, HD, KH, C::NCW, C::NPG, C::MERGE, NT>(
+    vx_attention_mfma_body<true, HD, KH, NCW, C::NPG, C::MERGE, NT>(
         q, M, n_past, n_ctx, n_heads, n_kv, cap, kc, vc, n_chunks, n_chunks_w, n_qg, part, qa);
 }
 
@@ -1252,26 +1277,26 @@ extern "C" size_t vxh_attention_rows_workspace_floats(int M, int n_ctx, int cap,
 
 // The fp32-MFMA kernels for a head size, cache precision and q source (q
 // rows, or the q|k|v sums of A when qkv is set).
-template <bool NT>
+template <bool NT, int NCW>
 static void vx_attention_mfma_launch(const float *q, bool qkv, const vx_qkv_args &A, int M, int n_past, int n_ctx,
                                      int n_heads, int n_kv_heads, int head_dim, int cap, float *kc, float *vc,
                                      int n_chunks, int n_chunks_w, int nqg, int grid, float *part, int kv_half,
                                      vxh_stream s)
 {
     if (kv_half && head_dim == 64)
-        vx_attention_mfma_qkv_kernel<64, true, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
+        vx_attention_mfma_qkv_kernel<64, true, NT, NCW><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
             nullptr, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
     else if (kv_half)
-        vx_attention_mfma_qkv_kernel<128, true, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
+        vx_attention_mfma_qkv_kernel<128, true, NT, NCW><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
             nullptr, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
     else if (head_dim == 64 && qkv)
-        vx_attention_mfma_qkv_kernel<64, false, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
+        vx_attention_mfma_qkv_kernel<64, false, NT, NCW><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
             nullptr, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
     else if (head_dim == 64)
         vx_attention_mfma_kernel<64, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
             q, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
     else if (qkv)
-        vx_attention_mfma_qkv_kernel<128, false, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
+        vx_attention_mfma_qkv_kernel<128, false, NT, NCW><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
             nullptr, M, n_past, n_ctx, n_heads, n_kv_heads, cap, kc, vc, n_chunks, n_chunks_w, nqg, part, A);
     else
         vx_attention_mfma_kernel<128, NT><<<grid, ATT_THREADS, 0, vxh_hs(s)>>>(
@@ -1361,11 +1386,14 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     vx_qkv_args none;
     memset(&none, 0, sizeof(none));
     const bool mfma = (head_dim == 64 || head_dim == 128) && (!qa || M <= VX_ATT_MFMA_MAX_M);
+    const int ncw = qa ? vx_att_ncw(head_dim, (size_t)n_kv_heads * head_dim * (kv_half ? 2 : 4),
+                                    (long)n_kv_heads * ((QM + 15) / 16) * ((ctx + 15) / 16))
+                       : 1;
     if (mfma) {
         // fp32-MFMA kernel: 4 wavefronts per workgroup, wch positions each
         int wch;
         bool merge;
-        vx_att_geom(head_dim, qa != nullptr, &wch, &merge);
+        vx_att_geom(head_dim, qa != nullptr, ncw, &wch, &merge);
         const int nw_w = (n_chunks_w * ACH + wch - 1) / wch;
         const int nqg = (QM + 15) / 16, ncg = (nw_w + 3) / 4;
         const int grid = n_kv_heads * nqg * ncg;
@@ -1374,12 +1402,20 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
         // non-temporal loads (a 7B target's 2048-position rows: 64 MB; a 1B
         // draft's: 4 MB)
         const bool nt = 2.0 * ctx * n_kv_heads * head_dim * (kv_half ? 2 : 4) > VX_KV_STREAM_BYTES;
-        if (nt)
-            vx_attention_mfma_launch<true>(q, qa != nullptr, A, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap, kc, vc,
-                                           n_chunks, n_chunks_w, nqg, grid, ws->part, kv_half, s);
-        else
-            vx_attention_mfma_launch<false>(q, qa != nullptr, A, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap, kc, vc,
-                                            n_chunks, n_chunks_w, nqg, grid, ws->part, kv_half, s);
+#define VX_CALL(NT_, NCW_)                                                                                       \
+    vx_attention_mfma_launch<NT_, NCW_>(q, qa != nullptr, A, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap, \
+                                        kc, vc, n_chunks, n_chunks_w, nqg, grid, ws->part, kv_half, s)
+        if (ncw == 1) {
+            if (nt) VX_CALL(true, 1);
+            else VX_CALL(false, 1);
+        } else if (ncw == 2) {
+            if (nt) VX_CALL(true, 2);
+            else VX_CALL(false, 2);
+        } else {
+            if (nt) VX_CALL(true, 4);
+            else VX_CALL(false, 4);
+        }
+#undef VX_CALL
     } else if (qa)
         vx_attention_kernel<true><<<n_kv_heads * n_chunks_w * n_qg, ATT_THREADS, lds, vxh_hs(s)>>>(
             nullptr, M, n_past, n_ctx, n_heads, n_kv_heads, head_dim, cap, kc, vc, n_chunks, n_chunks_w,
@@ -1393,7 +1429,7 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     if (mfma) {
         int wch;
         bool merge;
-        vx_att_geom(head_dim, qa != nullptr, &wch, &merge);
+        vx_att_geom(head_dim, qa != nullptr, ncw, &wch, &merge);
         const int nw = (n_chunks * ACH + wch - 1) / wch;
         n_chunks = merge ? (nw + 3) / 4 : nw;
     }
