@@ -1181,21 +1181,31 @@ __global__ __launch_bounds__(256) void vx_attention_join_kernel(const float *__r
     const int d4 = threadIdx.x % L4, g = (int)(i / QM), qi = (int)(i % QM), m = qi % M, head = g * G + qi / M;
     const size_t cstride = (size_t)QM * PART_STRIDE(HD);
     const float *pq = part + (size_t)g * n_seg * cstride + (size_t)qi * PART_STRIDE(HD);
-    float mx = -INFINITY;
-    for (int c = 0; c < n_seg; c++) mx = fmaxf(mx, pq[c * cstride]);
-    float l = 0.0f;
+    float mx = -INFINITY, l = 0.0f;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int c = 0; c < n_seg; c++) {
-        const float *pc = pq + c * cstride;
-        const float cm = pc[0];
-        if (cm == -INFINITY) continue;       // a segment past the query's positions: sums not written
-        const float f = expf(cm - mx);
-        const float4 v = *(const float4 *)(pc + 4 + 4 * d4);
-        l = fmaf(f, pc[1], l);
-        a.x = fmaf(f, v.x, a.x);
-        a.y = fmaf(f, v.y, a.y);
-        a.z = fmaf(f, v.z, a.z);
-        a.w = fmaf(f, v.w, a.w);
+    constexpr int NB = 4;                    // segments whose loads leave together
+    for (int c0 = 0; c0 < n_seg; c0 += NB) {
+        float cm[NB], cl[NB];
+        float4 ca[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const float *pc = pq + min(c0 + u, n_seg - 1) * cstride;
+            cm[u] = c0 + u < n_seg ? pc[0] : -INFINITY;
+            cl[u] = pc[1];
+            ca[u] = *(const float4 *)(pc + 4 + 4 * d4);
+        }
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            if (cm[u] == -INFINITY) continue;       // past the query's positions: sums not written
+            const float nm = fmaxf(mx, cm[u]);
+            const float fo = mx == -INFINITY ? 0.0f : expf(mx - nm), fn = expf(cm[u] - nm);
+            l = l * fo + cl[u] * fn;
+            a.x = a.x * fo + ca[u].x * fn;
+            a.y = a.y * fo + ca[u].y * fn;
+            a.z = a.z * fo + ca[u].z * fn;
+            a.w = a.w * fo + ca[u].w * fn;
+            mx = nm;
+        }
     }
     const float inv = 1.0f / (l + 1e-10f);
     *(float4 *)(out + (size_t)m * ld_out + (size_t)head * HD + 4 * d4) =
@@ -1248,8 +1258,11 @@ static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int *seg_t)
     return (n_t + *seg_t - 1) / *seg_t;
 }
 
-// up to this many segments are joined by one thread per four outputs, in turn
-#define VX_JOIN_SEGMENTS 32
+// up to this many segments are joined by one thread per four outputs (two round
+// trips); more of them come with few queries, where the combine kernel's 256
+// threads per query walk them at once (500 rows x 2 heads of 64 over 3500, 32
+// segments: 26 us, 42 with the join)
+#define VX_JOIN_SEGMENTS 8
 
 // What any batch of up to M rows over up to ctx positions needs: the chunk
 // kernels' partials where they run (VX_ATT_MFMA_MAX_M rows, or fewer scores
