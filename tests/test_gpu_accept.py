@@ -118,6 +118,35 @@ def test_sampler_matches_oracle(P, V, T, top_p, mc):
     assert ties <= 2
 
 
+@pytest.mark.parametrize("V", [1, 2, 63, 1024, 1025, 40000])
+@pytest.mark.parametrize("top_p", [1e-9, 0.3, 0.5, 0.9, 0.999999, 0.99999999])
+def test_nucleus_of_tied_logits(P, V, top_p):
+    """Logits of three values, so that the threshold falls among many equal
+    probabilities and the ties enter in index order.  The members are the
+    shortest run (by value, then index) whose mass reaches top_p: counted in
+    float64, give or take the rounding of V fp32 probabilities (each within
+    2^-21 of its value, so 2^-20 of the count and one token)."""
+    print(f"tied nucleus V={V} top_p={top_p}", flush=True)
+    rng = np.random.default_rng(V + int(top_p * 1000))
+    l = rng.choice([0.0, -0.75, -2.0], V).astype(np.float32)
+    tok, nuc = sample_gpu(P, l, 1.0, top_p, 0.37)
+    e = np.exp(l.astype(np.float64) - l.max())
+    p = e / e.sum()
+    order = np.lexsort((np.arange(V), -p))
+    need = int(np.searchsorted(np.cumsum(p[order]), top_p * (1 - 1e-12)) + 1)
+    tau, tie = nuc[2], int(nuc[3:4].view(np.int32)[0])
+    if tau < 0:
+        member = np.ones(V, bool)
+    else:
+        level = l[np.argmin(np.abs(p - tau))]      # the logit whose probability tau is
+        assert abs(p[l == level][0] - tau) <= 2.0 ** -20 * tau
+        member = (l > level) | ((l == level) & (np.arange(V) <= tie))
+    assert abs(int(member.sum()) - min(need, V)) <= 1 + V * 2.0 ** -20
+    assert member[tok]
+    got = member[order]
+    assert np.all(got[:-1] >= got[1:]), "members are a prefix of the order by value, then index"
+
+
 @pytest.mark.parametrize("V,T,top_p", [(32000, 0.8, 1.0), (1001, 0.0, 1.0), (5000, 0.7, 0.5), (40000, 1.0, 1.0)])
 def test_sample_keep_copies_the_row_and_draws_like_sample(P, V, T, top_p):
     """vxh_sample_keep = vxh_sample plus a copy of the row (register sampler:
