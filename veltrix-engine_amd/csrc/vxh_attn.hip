@@ -1243,16 +1243,20 @@ extern "C" size_t vxh_attention_workspace_floats(int M, int n_ctx, int cap, int 
 #define VX_ROWS_MIN_SCORES 1e6
 
 // Context segments of the prompt kernel, in whole tiles (*seg_t of them each):
-// 512 workgroups (two per CU) once a CU has 8 tiles or more to do, else 256:
-// 500 rows x 32 heads of 64 over 2036 positions 122 us at 256, 115 at 512;
-// 100 rows x 32 heads of 128 over 1100: 48 and 50.  At most 1024 positions a
-// segment: the workgroups of a long causal prompt end together.
-static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int *seg_t)
+// 512 workgroups once a CU has 8 tiles or more to do, else 256: 500 rows x 32
+// heads of 64 over 2036 positions 122 us at 256, 115 at 512; 100 rows x 32 heads
+// of 128 over 1100: 48 and 50.  At most 1024 positions a segment: the workgroups
+// of a long causal prompt end together.  At head_dim 128 two workgroups fit a
+// CU, so no count just above 512, which would leave a second round nearly
+// empty (1100 rows x 32 heads: 576 workgroups 187 us, 864 146; 300 x 28/4 over
+// 2300: 544 133, 476 127); at 64 three fit, and one segment more is as good.
+static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int head_dim, int *seg_t)
 {
     const int n_t = (ctx + AR_T - 1) / AR_T;
     const long wgs = (long)n_kv_heads * ((QM + AR_Q - 1) / AR_Q), target = wgs * n_t >= 2048 ? 512 : 256;
-    int n_seg = (int)((target + wgs - 1) / wgs);
+    int n_seg = (int)((head_dim == 64 ? target + wgs - 1 : target) / wgs);
     if (n_seg < (n_t + 31) / 32) n_seg = (n_t + 31) / 32;
+    if (head_dim != 64 && wgs * n_seg > 512 && wgs * n_seg < 768) n_seg++;
     if (n_seg > n_t) n_seg = n_t;
     *seg_t = (n_t + n_seg - 1) / n_seg;
     return (n_t + *seg_t - 1) / *seg_t;
@@ -1267,7 +1271,8 @@ static int vx_rows_segments(int n_kv_heads, int QM, int ctx, int *seg_t)
 // What any batch of up to M rows over up to ctx positions needs: the chunk
 // kernels' partials where they run (VX_ATT_MFMA_MAX_M rows, or fewer scores
 // than VX_ROWS_MIN_SCORES), the segments' elsewhere (at most 128 queries for
-// each of 512 workgroups and one more segment, or 1024 positions a segment).
+// each of 768 workgroups and one more segment, or 1024 positions a segment and
+// one more).
 extern "C" size_t vxh_attention_rows_workspace_floats(int M, int n_ctx, int cap, int n_heads, int n_kv_heads,
                                                       int head_dim)
 {
@@ -1276,7 +1281,7 @@ extern "C" size_t vxh_attention_rows_workspace_floats(int M, int n_ctx, int cap,
     const size_t ctx = cap > 0 && n_ctx > cap ? cap : n_ctx, q = (size_t)n_heads * M;
     const size_t few = (size_t)n_heads * VX_ATT_MFMA_MAX_M * ((ctx + ACH - 1) / ACH);
     const size_t small = (size_t)(VX_ROWS_MIN_SCORES / ACH) + 1 + q;
-    const size_t seg = 512 * AR_Q + q, lon = q * ((ctx + 1023) / 1024 + 1);
+    const size_t seg = 768 * AR_Q + q, lon = q * ((ctx + 1023) / 1024 + 1);
     size_t need = few > small ? few : small;
     if (seg > need) need = seg;
     if (lon > need) need = lon;
@@ -1367,7 +1372,7 @@ static int vx_attention_run(const float *q, const vx_qkv_args *qa, long n_clr, i
     const bool rows = !qa && !parts_only && (head_dim == 64 || head_dim == 128) && M > VX_ATT_MFMA_MAX_M &&
                       (double)n_heads * M * ctx >= VX_ROWS_MIN_SCORES;
     int seg_t = 0;
-    const int n_seg = rows ? vx_rows_segments(n_kv_heads, QM, ctx, &seg_t) : 0;
+    const int n_seg = rows ? vx_rows_segments(n_kv_heads, QM, ctx, head_dim, &seg_t) : 0;
     size_t need = (size_t)n_kv_heads * (rows && rows_ws ? n_seg : n_chunks) * QM * PART_STRIDE(head_dim);
     if (need > ws->part_floats)
         return vxh_fail(VXH_ERR_PARAM, "attention workspace too small (%zu floats needed)", need);

@@ -1,7 +1,8 @@
 // Prompt prefill at large M: the reference runs the prompt one token per
 // forward (src/speculative.c:100-107, src/model.c:450-616); here a chunk of
-// up to a few hundred prompt rows runs as one batch.
+// up to a few thousand prompt rows runs as one batch.
 //
+//   vx_pf_panel_kernel   rows, their RMSNorm or SwiGLU as the GEMM's operand
 //   vx_pf_gemm_kernel    Y = X W^T (+ R) for M rows, compute-bound MFMA tiles
 //   vx_pf_rope_kv_kernel RoPE of q|k rows and the k/v cache store (fp32 rows)
 //   vx_pf_swiglu_kernel  h = |silu(g)| < thr ? 0 : silu(g) * u
