@@ -118,7 +118,7 @@ def test_sampler_matches_oracle(P, V, T, top_p, mc):
     assert ties <= 2
 
 
-@pytest.mark.parametrize("V", [1, 2, 63, 1024, 1025, 40000])
+@pytest.mark.parametrize("V", [1, 2, 63, 1024, 1025, 32768, 32769, 40000])
 @pytest.mark.parametrize("top_p", [1e-9, 0.3, 0.5, 0.9, 0.999999, 0.99999999])
 def test_nucleus_of_tied_logits(P, V, top_p):
     """Logits of three values, so that the threshold falls among many equal

@@ -280,6 +280,14 @@ __device__ bool vx_wg_tau(int V, uint64_t TP, PF P, uint64_t *hist, uint64_t *ws
     return true;
 }
 
+// LP: the probabilities of a row of up to SB * SE entries in LDS, evaluated
+// once (the histograms, ties and draw read them about ten times); one word of
+// padding per 32 entries keeps a thread's contiguous entries off one bank.
+// top_p 0.9, 32000 entries: draw, statistics and decision 124 -> 87 us.
+#define SE 32                            // entries per thread that are held on chip
+#define SP_WORDS (SB * SE + SB * SE / 32)
+
+template <bool LP>
 __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__ l, int V, float T,
                                                        float top_p, const float *__restrict__ u,
                                                        int *__restrict__ token_out,
@@ -292,6 +300,7 @@ __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__
     __shared__ uint64_t s_above;
     __shared__ uint32_t s_bin;
     __shared__ int res;
+    __shared__ float s_p[LP ? SP_WORDS : 1];
 
     float bv = -INFINITY;
     int bi = 0x7fffffff;
@@ -313,6 +322,14 @@ __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__
     for (int v = threadIdx.x; v < V; v += SB) s += expf((l[v] - mx) / T);
     s = vx_wg_sum(s, redv);
     const float inv = 1.0f / (s + 1e-30f);
+    if constexpr (LP) {
+        for (int v = threadIdx.x; v < V; v += SB) s_p[v + (v >> 5)] = vx_prob(l, v, mx, inv, T);
+        __syncthreads();
+    }
+    auto P = [&](int v) -> float {
+        if constexpr (LP) return s_p[v + (v >> 5)];
+        else return vx_prob(l, v, mx, inv, T);
+    };
 
     float tau = -1.0f;
     int tie_cut = V - 1;
@@ -323,7 +340,7 @@ __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__
         const uint64_t TP = tpu < 1.0 ? 1ull : (uint64_t)tpu;
         uint64_t gt = 0;
         tau = 0.0f;      // all the mass is below TP: every token
-        vx_wg_tau(V, TP, [&](int v) { return vx_prob(l, v, mx, inv, T); }, scan, red64, &s_bin, &s_above, &tau, &gt);
+        vx_wg_tau(V, TP, P, scan, red64, &s_bin, &s_above, &tau, &gt);
         const uint64_t pt = vx_fixed32(tau);
         if (pt == 0 || gt >= TP) {
             tie_cut = V - 1;   // cannot happen for tau > 0; keep every tie
@@ -332,13 +349,13 @@ __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__
             const uint64_t need_units = TP - gt;
             const uint64_t j = (need_units + pt - 1) / pt;    // number of ties needed
             tie_cut = vx_wg_find_prefix(V, j, [&](int v) -> uint64_t {
-                return vx_prob(l, v, mx, inv, T) == tau ? 1ull : 0ull;
+                return P(v) == tau ? 1ull : 0ull;
             }, scan, &res);
         }
         if (tau <= 0.0f) { tau = -1.0f; tie_cut = V - 1; }
     }
     auto member_w = [&](int v) -> uint64_t {
-        float p = vx_prob(l, v, mx, inv, T);
+        float p = P(v);
         bool in = tau < 0.0f || p > tau || (p == tau && v <= tie_cut);
         return in ? vx_fixed32(p) : 0ull;
     };
@@ -361,8 +378,6 @@ __global__ __launch_bounds__(SB) void vx_sample_kernel(const float *__restrict__
 // search uses per-wavefront totals and one lane scan in the wavefront where
 // the threshold lands (no passes over the row).  Same arithmetic as
 // vx_sample_kernel with top_p = 1.
-#define SE 32
-
 __device__ __forceinline__ uint64_t vx_shfl_u64(uint64_t v, int src)
 {
     const uint32_t lo = __shfl((int)(uint32_t)v, src, 64), hi = __shfl((int)(uint32_t)(v >> 32), src, 64);
@@ -547,7 +562,10 @@ extern "C" int vxh_sample_keep(const float *l, int V, float T, float top_p, cons
         vx_sample_reg_kernel<<<1, SB, 0, vxh_hs(s)>>>(l, V, T, u_dev, token_out, nuc, keep);
     } else {
         if (keep) VXH_CHECK(hipMemcpyAsync(keep, l, sizeof(float) * (size_t)V, hipMemcpyDeviceToDevice, vxh_hs(s)));
-        vx_sample_kernel<<<1, SB, 0, vxh_hs(s)>>>(l, V, T, top_p, u_dev, token_out, nuc);
+        if (top_p < 1.0f && V <= SB * SE)
+            vx_sample_kernel<true><<<1, SB, 0, vxh_hs(s)>>>(l, V, T, top_p, u_dev, token_out, nuc);
+        else
+            vx_sample_kernel<false><<<1, SB, 0, vxh_hs(s)>>>(l, V, T, top_p, u_dev, token_out, nuc);
     }
     VXH_LAUNCHED();
     return VXH_OK;
