@@ -402,7 +402,9 @@ int vxh_rope_kv_norm(double *qkv, int ld_qkv, int M, int n_past, int n_ctx, int 
  * (src/model.c:300-338): row m reads positions [0, min(pos_m + 1, cap)),
  * head h uses kv head h*n_kv/n_heads, softmax with 1/(sum + 1e-10).  Two
  * launches: per-chunk partial softmax, then the cross-chunk combine; the
- * partials live in ws->part.  head_dim: a multiple of 4, at most 128. */
+ * partials live in ws->part.  head_dim: a multiple of 4, at most 128.  Cache
+ * rows past the last position any of the M rows attends may hold anything, NaN
+ * included (here and in every attention entry point below). */
 int vxh_attention(const float *q, int M, int n_past, int n_ctx, int n_heads, int n_kv_heads,
                   int head_dim, int cap, const float *k_cache_layer,
                   const float *v_cache_layer, float *out, int ld_out,

@@ -463,6 +463,89 @@ def test_attention_qkv_walks_several_chunks(P, H, KV, hd, M, n_past, n_ctx, cap)
     test_attention_qkv_matches_rope_then_attention(P, H, KV, hd, M, n_past, n_ctx, cap, True)
 
 
+def att_end(M, n_past, n_ctx, cap):
+    """One past the last position any of the rows attends."""
+    end = min(n_past + M, n_ctx)
+    return min(end, cap) if cap else end
+
+
+def qkv_chunks(H, KV, hd, M, n_past, n_ctx, cap, half):
+    """16-position chunks a wavefront of the q|k|v kernel walks (the rule of the dispatch)."""
+    row, ctx = KV * hd * (2 if half else 4), att_end(M, n_past, n_ctx, cap)
+    waves = KV * ((H // KV * M + 15) // 16) * ((ctx + 15) // 16)
+    if row >= 16384:
+        return 1
+    two, four = (1200 if hd == 64 else 3500), (6000 if hd == 64 or row >= 8192 else 3500)
+    return 4 if waves >= four else 2 if waves >= two else 1
+
+
+# (q source, chunks per wavefront: None where another kernel runs, heads ...)
+UNATTENDED = [
+    ("qkv", 1, 28, 4, 128, 9, 300, 400, 0), ("qkv", 2, 16, 16, 128, 9, 3600, 3700, 0),
+    ("qkv", 4, 28, 4, 128, 9, 8151, 8192, 0), ("qkv", 4, 28, 4, 128, 9, 8000, 8192, 4099),
+    ("qkv", 4, 28, 4, 128, 9, 4095, 4200, 4099),      # the cap ends inside the new rows
+    ("qkv", 1, 32, 4, 64, 1, 130, 200, 0), ("qkv", 2, 32, 4, 64, 9, 1040, 1200, 0),
+    ("qkv", 4, 16, 8, 64, 9, 6149, 6300, 0), ("qkv", 1, 8, 2, 128, 3, 0, 64, 0),
+    ("f16", 1, 32, 4, 64, 9, 75, 200, 0), ("f16", 2, 32, 32, 128, 2, 1800, 1900, 0),
+    ("f16", 4, 28, 4, 128, 9, 8151, 8192, 0), ("f16", 4, 32, 32, 64, 16, 3035, 3200, 0),
+    ("qkv", None, 8, 2, 32, 5, 70, 256, 40), ("qkv", None, 8, 2, 64, 20, 70, 256, 0),   # LDS kernel
+    ("q", None, 32, 4, 64, 1, 130, 200, 0), ("q", None, 8, 8, 128, 9, 300, 512, 0),
+    ("q", None, 4, 4, 64, 300, 640, 940, 700), ("q", None, 8, 2, 96, 9, 70, 256, 0),
+    ("q", None, 8, 2, 128, 384, 500, 1000, 0)]        # prompt kernel
+
+
+@pytest.mark.parametrize("src,chunks,H,KV,hd,M,n_past,n_ctx,cap", UNATTENDED)
+def test_attention_ignores_rows_no_query_attends(P, src, chunks, H, KV, hd, M, n_past, n_ctx, cap):
+    """What the cache holds past the batch's last attended position reaches no
+    output: NaN there (K and V) gives the bits that ordinary rows give, at
+    every count of chunks per wavefront, for the LDS and the prompt kernel and
+    both cache precisions."""
+    print(f"unattended rows {src} H={H} KV={KV} hd={hd} M={M} n_past={n_past} n_ctx={n_ctx} cap={cap}", flush=True)
+    bind_attention(P)
+    if chunks:
+        assert qkv_chunks(H, KV, hd, M, n_past, n_ctx, cap, src == "f16") == chunks
+    P.vxh_attention_qkv_f16.argtypes = P.vxh_attention_qkv.argtypes
+    rng = np.random.default_rng(H * 3 + hd + M + n_past)
+    qd, kvd = H * hd, KV * hd
+    ld = qd + 2 * kvd
+    qv = rng.normal(0, 1, (M, ld))
+    n_pos = max(n_past + M, n_ctx) + 1
+    ang = np.arange(n_pos)[:, None] / np.power(10000.0, np.arange(hd // 2) * 2.0 / hd)[None, :]
+    dcs, dsn = N.DevBuf(P, np.cos(ang).astype(np.float32)), N.DevBuf(P, np.sin(ang).astype(np.float32))
+    typ = np.float16 if src == "f16" else np.float32
+    cache = rng.normal(0, 1, (2, n_ctx, kvd)).astype(typ)
+    end = att_end(M, n_past, n_ctx, cap)
+    ws = Workspace()
+    assert P.vxh_workspace_alloc(C.byref(ws), 32, P.vxh_attention_workspace_floats(M, n_ctx, cap, H, KV, hd)) == 0
+    outs = []
+    for fill in (None, np.nan):
+        c = cache.copy()
+        if fill is not None:
+            c[:, end:] = fill
+        bits = np.uint16 if src == "f16" else np.float32
+        dk, dv = N.DevBuf(P, c[0].view(bits)), N.DevBuf(P, c[1].view(bits))
+        dout = N.DevBuf(P, np.zeros((M, qd), np.float32))
+        if src == "q":
+            dq = N.DevBuf(P, qv[:, :qd].astype(np.float32))
+            rc = P.vxh_attention(dq.ptr, M, n_past, n_ctx, H, KV, hd, cap, dk.ptr, dv.ptr, dout.ptr, qd, C.byref(ws),
+                                 None)
+        else:
+            dq = N.DevBuf(P, qv)
+            f = P.vxh_attention_qkv if src == "qkv" else P.vxh_attention_qkv_f16
+            rc = f(dq.ptr, ld, None, 0, None, None, None, dcs.ptr, dsn.ptr, n_pos, M, n_past, n_ctx, H, KV, hd, cap,
+                   dk.ptr, dv.ptr, dout.ptr, qd, C.byref(ws), None)
+        assert rc == 0, P.vxh_last_error()
+        assert P.vxh_stream_sync(None) == 0
+        outs.append(dout.get(np.float32, M * qd))
+        for b in (dk, dv, dout, dq):
+            b.free()
+    P.vxh_workspace_free(C.byref(ws))
+    dcs.free()
+    dsn.free()
+    assert np.isfinite(outs[0]).all()
+    assert np.array_equal(outs[0], outs[1])
+
+
 def test_attention_qkv_rejects_clamped_batches(P):
     bind_attention(P)
     ws = Workspace()

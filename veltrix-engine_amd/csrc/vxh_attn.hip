@@ -124,6 +124,20 @@ __device__ __forceinline__ float4 vx_qkv4(const vx_qkv_args &a, int m, int col, 
     return make_float4(o0.x, o0.y, o1.x, o1.y);
 }
 
+// v where ok, else zeros (per component: a select of whole float4 array
+// elements becomes a select of their addresses and puts the array in scratch)
+__device__ __forceinline__ float4 vx_keep4(bool ok, float4 v)
+{
+    return make_float4(ok ? v.x : 0.0f, ok ? v.y : 0.0f, ok ? v.z : 0.0f, ok ? v.w : 0.0f);
+}
+
+// One past the last position any of the M rows attends.
+__device__ __forceinline__ int vx_att_end(int n_past, int M, int n_ctx, int cap)
+{
+    const int end = min(n_past + M, n_ctx);
+    return cap > 0 && end > cap ? cap : end;
+}
+
 template <bool QKV>
 __global__ __launch_bounds__(ATT_THREADS) void vx_attention_kernel(
     const float *__restrict__ q, int M, int n_past, int n_ctx, int n_heads, int n_kv, int hd,
@@ -151,7 +165,10 @@ __global__ __launch_bounds__(ATT_THREADS) void vx_attention_kernel(
     const float scale = 1.0f / sqrtf((float)hd);
 
     // K/V chunk: ACH*hd/4 float4 each, at most 4 per thread; rows past the
-    // cache end read as zeros (their scores are masked below)
+    // cache end read as zeros (their scores are masked below), V rows from the
+    // batch's last attended position on too: their probability is 0, and 0
+    // times what the cache holds there may be NaN
+    const int t_end = vx_att_end(n_past, M, n_ctx, cap);
     constexpr int KV4 = ACH * ATT_MAX_HD / 4 / ATT_THREADS;
     float4 kr[KV4], vr[KV4];
     const int qd = n_heads * hd, half = hd / 2;
@@ -182,6 +199,7 @@ __global__ __launch_bounds__(ATT_THREADS) void vx_attention_kernel(
             kr[j] = ok ? *(const float4 *)(kc + off) : make_float4(0.f, 0.f, 0.f, 0.f);
             vr[j] = ok ? *(const float4 *)(vc + off) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
+        vr[j] = vx_keep4(pos < t_end, vr[j]);
     }
     if (ch >= n_chunks) return;
     for (int i = threadIdx.x; i < nq * hd4; i += ATT_THREADS) {
@@ -322,13 +340,6 @@ __device__ __forceinline__ void vx_qkv4_items(const vx_qkv_args &a, const int ro
 
 #define VX_ATT_MFMA_MAX_M VXH_ATTN_QKV_FAST_ROWS   // rows of a forward the QKV variant takes
 
-// v where ok, else zeros (per component: a select of whole float4 array
-// elements becomes a select of their addresses and puts the array in scratch)
-__device__ __forceinline__ float4 vx_keep4(bool ok, float4 v)
-{
-    return make_float4(ok ? v.x : 0.0f, ok ? v.y : 0.0f, ok ? v.z : 0.0f, ok ? v.w : 0.0f);
-}
-
 // KV cache rows in fp32 (KH = false, the reference's cache) or IEEE fp16
 // (KH = true, a flagged mode: round to nearest even on store, exact widening
 // on load).  i is an element index, a multiple of 4.
@@ -446,10 +457,12 @@ __device__ __forceinline__ void vx_attention_mfma_body(
 
     // K rows of positions tc + 16 pg + n (dims 16 j + 4 r .. + 3) and V rows
     // of positions tc + 16 pg + 4 r + s (dims 64 u + 4 n .. + 3) of chunk tc
-    // from the cache; positions past the cache end read as zeros (with one
-    // chunk per wavefront only a chunk that reaches past it -- wavefront-
-    // uniform -- runs the selects; a branch between a multi-chunk wavefront's
-    // loads would wait for the next chunk's K before this chunk's P.V).
+    // from the cache; positions past the cache end, and V rows from the last
+    // attended position on (probability 0, but 0 times what the cache holds
+    // there may be NaN), read as zeros (with one chunk per wavefront only a
+    // chunk that reaches past the end -- wavefront-uniform -- runs the
+    // selects; a branch between a multi-chunk wavefront's loads would wait
+    // for the next chunk's K before this chunk's P.V).
     // Offsets are 32-bit element indices from the layer's cache base.
     float4 kr[NPG][NJ], vr[NPG][4][NV4];
     const uint32_t head0 = (uint32_t)(g * HD), ukvd = (uint32_t)kvd;
@@ -470,6 +483,7 @@ __device__ __forceinline__ void vx_attention_mfma_body(
             }
         }
     };
+    const int t_end = vx_att_end(n_past, M, n_ctx, cap);
     auto load_v = [&](int tc) {
 #pragma unroll
         for (int pg = 0; pg < NPG; pg++)
@@ -480,12 +494,12 @@ __device__ __forceinline__ void vx_attention_mfma_body(
 #pragma unroll
                 for (int u = 0; u < NV4; u++) vr[pg][st][u] = vx_kv_load4<KH, NT>(vc, ov + 64 * u);
             }
-        if (NCW > 1 || tc + 16 * NPG > n_ctx) {
+        if (NCW > 1 || tc + 16 * NPG > t_end) {
 #pragma unroll
             for (int pg = 0; pg < NPG; pg++)
 #pragma unroll
                 for (int st = 0; st < 4; st++) {
-                    const bool okv = tc + 16 * pg + 4 * r + st < n_ctx;
+                    const bool okv = tc + 16 * pg + 4 * r + st < t_end;
 #pragma unroll
                     for (int u = 0; u < NV4; u++) vr[pg][st][u] = vx_keep4(okv, vr[pg][st][u]);
                 }
@@ -687,8 +701,8 @@ __device__ __forceinline__ void vx_attention_mfma_body(
             for (int pg = 0; pg < NPG; pg++)
 #pragma unroll
                 for (int st = 0; st < 4; st++) {
-                    const int mv = new_row(tc + 16 * pg + 4 * r + st);
-                    if (mv >= 0)
+                    const int pv = tc + 16 * pg + 4 * r + st, mv = new_row(pv);
+                    if (mv >= 0 && pv < t_end)
 #pragma unroll
                         for (int u = 0; u < NV4; u++) vr[pg][st][u] = s_new[(mv * 2 + 1) * (HD / 4) + n + 16 * u];
                 }
