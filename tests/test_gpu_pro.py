@@ -12,6 +12,7 @@ fp64 sum; products within 1e-4 + 1e-3*|oracle| or closer to the fp64 exact
 value than the oracle is (the `parity` helper); cleared ranges all zero.
 """
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -635,6 +636,7 @@ def test_pro_attn_combines_partials(P, H, KV, hd, M, typ):
     (8, 8, 128, 16, 100, 512, 4096),      # 16 query vectors per kv head
     (16, 2, 32, 3, 90, 256, 4096),        # head_dim 32: 32-position chunks
     (8, 2, 128, 64, 300, 512, 200),       # prompt-prefill batch: 64 rows, cap inside a two-chunk wavefront
+    (4, 4, 64, 300, 640, 940, 700),       # 300 rows below the prompt kernel's range, cap reached inside the batch
     (32, 32, 64, 2, 2100, 2304, 4096),    # 34 MB of cache rows: read with non-temporal loads
     (8, 2, 128, 9, 30000, 32768, 0),      # 32K context, no cap: ~940 chunk partials per query
     (8, 1, 64, 1, 32760, 32768, 0),       # the last positions of a 32K cache, one row
@@ -696,44 +698,77 @@ def test_pro_attn_reads_no_head_past_k(P, H, KV, hd, M, after):
     P.vxh_qmat_free(C.byref(q))
 
 
-@pytest.mark.parametrize("H,KV,hd,M,n_past,n_ctx,cap", [
-    (32, 32, 64, 17, 1830, 1847, 0),      # 17 queries per kv head: one wavefront of four at work
-    (32, 32, 64, 33, 992, 1100, 0),       # a second wavefront with one query; positions end on a tile edge
-    (8, 2, 128, 97, 1200, 1500, 0),       # four query groups, the last of four queries
-    (7, 1, 128, 150, 1100, 1300, 1000),   # seven heads per kv head, cap below every row
-    (4, 4, 64, 300, 640, 940, 700),       # cap reached inside the batch
-    (4, 1, 128, 33, 8100, 8133, 0),       # segments of 16 tiles and a short last one
-    (16, 2, 64, 257, 0, 300, 0),          # empty cache: segments past the first rows' positions
-    (2, 1, 128, 600, 500, 1000, 0),       # rows past the context clamp to its last position
-    (8, 8, 128, 384, 0, 384, 0)])
-def test_prompt_attention_matches_reference(P, H, KV, hd, M, n_past, n_ctx, cap):
+def bind_rows(P):
+    i = C.c_int
+    P.vxh_attention_rows.argtypes = [vp, i, i, i, i, i, i, i, vp, vp, vp, i, C.POINTER(Workspace), vp]
+    P.vxh_attention_rows_workspace_floats.restype = C.c_size_t
+    P.vxh_attention_rows_workspace_floats.argtypes = [i, i, i, i, i, i]
+
+
+def rows_floats_needed(P, H, KV, hd, M, n_past, n_ctx, cap):
+    """Workspace floats a call of vxh_attention_rows takes, from its refusal
+    of an empty workspace (checked before anything is launched)."""
+    rc = P.vxh_attention_rows(None, M, n_past, n_ctx, H, KV, hd, cap, None, None, None, H * hd, C.byref(Workspace()),
+                              None)
+    m = re.search(r"\((\d+) floats needed\)", P.vxh_last_error().decode())
+    assert rc != 0 and m, P.vxh_last_error()
+    return int(m.group(1))
+
+
+# heads ..., context segments
+@pytest.mark.parametrize("H,KV,hd,M,n_past,n_ctx,cap,segs", [
+    (32, 32, 64, 17, 1830, 1847, 0, 8),       # 17 queries per kv head: one wavefront of four at work
+    (32, 32, 64, 33, 992, 1100, 0, 7),        # a second wavefront with one query; positions end on a tile edge
+    (8, 2, 128, 97, 1200, 1500, 0, 21),       # four query groups, the last of four queries
+    (7, 1, 128, 150, 1100, 1300, 1000, 16),   # seven heads per kv head, cap below every row
+    (8, 8, 64, 300, 640, 940, 700, 11),       # cap reached inside the batch
+    (4, 1, 128, 33, 8100, 8133, 0, 128),      # 255 tiles: the last segment has one
+    (8, 8, 128, 1000, 3000, 4000, 0, 8),      # segments of 16 tiles and a last one of 13
+    (16, 2, 64, 257, 0, 300, 0, 5),           # empty cache: segments past the first rows' positions
+    (2, 1, 128, 600, 500, 1000, 0, 16),       # rows past the context clamp to its last position
+    (8, 8, 128, 384, 0, 384, 0, 6),
+    (48, 48, 128, 700, 0, 700, 0, 1),         # one segment: the kernel writes the rows itself
+    (128, 128, 64, 500, 0, 500, 0, 1),
+    (32, 32, 128, 1100, 0, 1100, 0, 3)])      # two segments would be 576 workgroups: three
+@pytest.mark.parametrize("entry", ["vxh_attention", "vxh_attention_rows"])
+def test_prompt_attention_matches_reference(P, entry, H, KV, hd, M, n_past, n_ctx, cap, segs):
     """The prompt kernel (128 queries per workgroup) against float64 softmax
-    attention, with NaN in the cache rows no query attends.  Bound: a score
+    attention, with NaN in the cache rows no query attends, on exactly the
+    workspace its entry point asks for (what follows it stays).  Bound: a score
     is an fp32 sum of hd products (at most hd/4 + 8 roundings of its sum of
     magnitudes, 2^-24 each), its exponential carries that error and 4 more
     roundings, and each output sum rounds once per position of a tile and
     twice per tile or segment (64 in all), relative to sum p |v|."""
-    print(f"prompt attention H={H} KV={KV} hd={hd} M={M} n_past={n_past} n_ctx={n_ctx} cap={cap}", flush=True)
+    print(f"prompt attention {entry} H={H} KV={KV} hd={hd} M={M} n_past={n_past} n_ctx={n_ctx} cap={cap}", flush=True)
     bind_attention(P)
+    bind_rows(P)
+    end = att_end(M, n_past, n_ctx, cap)
+    assert M > 16 and H * M * end >= 1e6, "takes the prompt kernel"
+    assert rows_floats_needed(P, H, KV, hd, M, n_past, n_ctx, cap) == segs * H * M * (hd + 4)
     rng = np.random.default_rng(H + KV * 5 + hd + M + n_past)
     qd, kvd = H * hd, KV * hd
     qv = rng.normal(0, 1.0, (M, qd)).astype(np.float32)
     kc = rng.normal(0, 1.0, (n_ctx, kvd)).astype(np.float32)
     vc = rng.normal(0, 1.0, (n_ctx, kvd)).astype(np.float32)
-    end = min(n_past + M, n_ctx, cap or n_ctx)
     kc[end:] = np.nan
     vc[end:] = np.nan
     dq, dk, dv = N.DevBuf(P, qv), N.DevBuf(P, kc), N.DevBuf(P, vc)
     dout = N.DevBuf(P, np.zeros((M, qd), np.float32))
-    ws = Workspace()
-    assert P.vxh_workspace_alloc(C.byref(ws), 32, P.vxh_attention_workspace_floats(M, n_ctx, cap, H, KV, hd)) == 0
-    rc = P.vxh_attention(dq.ptr, M, n_past, n_ctx, H, KV, hd, cap, dk.ptr, dv.ptr, dout.ptr, qd, C.byref(ws), None)
+    nf = getattr(P, entry + "_workspace_floats")(M, n_ctx, cap, H, KV, hd)
+    part = N.DevBuf(P, nbytes=4 * (nf + 256))
+    after = vp(part.ptr.value + 4 * nf)
+    canary = np.full(256, 0x5AC3F00D, np.uint32)
+    assert P.vxh_upload(after, canary.ctypes.data_as(vp), canary.nbytes, None) == 0
+    ws = Workspace(part=part.ptr, part_floats=nf)
+    rc = getattr(P, entry)(dq.ptr, M, n_past, n_ctx, H, KV, hd, cap, dk.ptr, dv.ptr, dout.ptr, qd, C.byref(ws), None)
     assert rc == 0, P.vxh_last_error()
     assert P.vxh_stream_sync(None) == 0
     got = dout.get(np.float32, M * qd).reshape(M, qd)
-    P.vxh_workspace_free(C.byref(ws))
-    for b in (dq, dk, dv, dout):
+    left = np.zeros_like(canary)
+    assert P.vxh_download(left.ctypes.data_as(vp), after, left.nbytes, None) == 0
+    for b in (dq, dk, dv, dout, part):
         b.free()
+    assert np.array_equal(left, canary)
     cs = np.minimum(np.minimum(n_past + np.arange(M), n_ctx - 1) + 1, cap or n_ctx)
     dead = np.arange(end)[None, :] >= cs[:, None]
     for h in range(H):
@@ -745,8 +780,8 @@ def test_prompt_attention_matches_reference(P, H, KV, hd, M, n_past, n_ctx, cap)
         p = np.exp(s - s.max(axis=1, keepdims=True))
         p /= p.sum(axis=1, keepdims=True) + 1e-10
         rel = 2.0 ** -24 * (2 * (hd / 4 + 8) * mag + 4 + 64)
-        bad = np.abs(got[:, h * hd:(h + 1) * hd] - p @ Vv) > rel[:, None] * (p @ np.abs(Vv))
-        assert not bad.any(), (h, np.argwhere(bad)[:4])
+        good = np.abs(got[:, h * hd:(h + 1) * hd] - p @ Vv) <= rel[:, None] * (p @ np.abs(Vv))   # false for NaN
+        assert good.all(), (h, np.argwhere(~good)[:4])
 
 
 def attention_ref(qv, kc, vc, H, KV, hd, n_past, n_ctx, cap):

@@ -215,3 +215,42 @@ def test_parity_helper_row_budget():
     gpu = oracle + 2e-4                                 # within the bar wherever |oracle| > 0.1
     gpu[:, 0] = oracle[:, 0] + 1.0                      # a dropped term
     assert not N.parity(gpu, oracle, exact)[0]
+
+
+def test_attention_workspaces_hold_what_calls_take(P):
+    """The floats a call takes (its refusal of an empty workspace names them,
+    before any GPU call) never exceed what the workspace functions return for
+    the same or a larger number of rows."""
+    i, vp = C.c_int, C.c_void_p
+
+    class Workspace(C.Structure):
+        _fields_ = [("acc", vp), ("acc_elems", C.c_size_t), ("part", vp), ("part_floats", C.c_size_t)]
+
+    for n in ("vxh_attention", "vxh_attention_rows"):
+        getattr(P, n).argtypes = [vp, i, i, i, i, i, i, i, vp, vp, vp, i, C.POINTER(Workspace), vp]
+        f = getattr(P, n + "_workspace_floats")
+        f.restype, f.argtypes = C.c_size_t, [i, i, i, i, i, i]
+    P.vxh_last_error.restype = C.c_char_p
+    rng = np.random.default_rng(11)
+    spread = lambda lo, hi: int(round(lo * (hi / lo) ** rng.random()))
+    seen = set()
+    for _ in range(20000):
+        kv = spread(1, 64)
+        H, hd = kv * int(rng.choice([1, 2, 3, 4, 7, 8])), int(rng.choice([32, 64, 96, 128]))
+        n_ctx = spread(1, 32768)
+        most = spread(1, 2048)                    # rows the workspace is made for
+        M = most if rng.random() < 0.3 else int(rng.integers(1, most + 1))
+        n_past = int(rng.integers(0, n_ctx + 3))
+        cap = int(rng.choice([0, 0, 4096, spread(1, 40000)]))
+        if n_ctx * kv * hd * 4 > 0xFFFFFFFF:
+            continue
+        for n in ("vxh_attention", "vxh_attention_rows"):
+            have = getattr(P, n + "_workspace_floats")(most, n_ctx, cap, H, kv, hd)
+            rc = getattr(P, n)(None, M, n_past, n_ctx, H, kv, hd, cap, None, None, None, H * hd,
+                               C.byref(Workspace()), None)
+            m = re.search(rb"\((\d+) floats needed\)", P.vxh_last_error())
+            assert rc != 0 and m, P.vxh_last_error()
+            need = int(m.group(1))
+            assert need <= have, (n, H, kv, hd, M, most, n_past, n_ctx, cap, need, have)
+            seen.add((n, need % (H * M * (hd + 4)) == 0 and need // (H * M * (hd + 4)) == 1))
+    assert ("vxh_attention_rows", True) in seen       # one segment (or chunk) was among them
