@@ -59,8 +59,10 @@ typedef struct {
                                   then hold halves                                    */
     int prefill_min_rows;      /* prompt chunks of at least this many rows whose
                                   positions fit the context run as one large-M
-                                  batch (up to 2048 rows; exact Q4_0 kernel, fp32
-                                  cache); 0 = never.  Default 48               */
+                                  batch (up to 2048 rows, 512 at head sizes other
+                                  than 64 and 128, fewer where the device has no
+                                  room; exact Q4_0 kernel, fp32 cache); 0 = never.
+                                  Default 48                                   */
 } vx_model_options;
 
 #define VX_FUSED_NONE 0        /* separate row kernels (11 launches per layer)          */

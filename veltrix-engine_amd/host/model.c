@@ -1187,31 +1187,49 @@ static vx_error pf_alloc_rows(vx_dev *d, int rows)
     return e;
 }
 
-/* Buffers for a chunk of P rows (grown in steps of VX_PF_GRAIN, up to
- * VX_PF_ROWS); where the device has no room for them, or the attention keeps a
- * partial per 32 positions (other head sizes), VX_PF_GRAIN rows. */
+/* The buffers fit the present cache and cap (the workspace is sized for both). */
+static int pf_sized(const vx_dev *d)
+{
+    return d->pf_rows && d->pf_ws_ctx == d->n_ctx_alloc && d->pf_ws_cap == d->opt.attn_cap;
+}
+
+/* Rows of the largest chunk: VX_PF_ROWS, VX_PF_GRAIN where the attention keeps
+ * a partial per 32 positions (other head sizes), or what the device was found
+ * to have room for at this cache size and cap. */
+static int pf_most(const vx_dev *d)
+{
+    const int most = d->hd == 64 || d->hd == 128 ? VX_PF_ROWS : VX_PF_GRAIN;
+    return pf_sized(d) && d->pf_limit && d->pf_limit < most ? d->pf_limit : most;
+}
+
+/* Buffers for a chunk of P <= pf_most(d) rows, grown in steps of VX_PF_GRAIN;
+ * fewer rows, down to VX_PF_GRAIN, where the device has no room for them.  What
+ * did not fit is not tried again until the cache or the cap changes. */
 static vx_error pf_alloc(vx_dev *d, int P)
 {
-    int R = (P + VX_PF_GRAIN - 1) / VX_PF_GRAIN * VX_PF_GRAIN;
-    const int most = d->hd == 64 || d->hd == 128 ? VX_PF_ROWS : VX_PF_GRAIN;
-    if (R > most) R = most;
-    if (d->pf_rows >= R) {
-        if (d->pf_ws_ctx == d->n_ctx_alloc && d->pf_ws_cap == d->opt.attn_cap) return VX_OK;
-        /* a cache allocated again for another n_ctx, or another cap: the
-         * attention workspace is sized for both */
-        TRY(vxh_stream_sync(d->stream));
-        vxh_workspace_free(&d->pf_ws);
-        d->pf_ws_ctx = -1;
-        return pf_ws_alloc(d, d->pf_rows);
-    }
+    const int R = (P + VX_PF_GRAIN - 1) / VX_PF_GRAIN * VX_PF_GRAIN;
+    if (pf_sized(d) && d->pf_rows >= R) return VX_OK;
+    int limit = pf_sized(d) ? d->pf_limit : 0;
     if (d->pf_rows) TRY(vxh_stream_sync(d->stream));
-    pf_free(d);
-    vx_error e = pf_alloc_rows(d, R);
-    if (e != VX_OK && R > VX_PF_GRAIN) {
-        pf_free(d);
-        e = pf_alloc_rows(d, VX_PF_GRAIN);
+    if (d->pf_rows >= R) {
+        /* a cache allocated again for another n_ctx, or another cap */
+        vxh_workspace_free(&d->pf_ws);
+        if (pf_ws_alloc(d, d->pf_rows) == VX_OK) {
+            d->pf_limit = 0;
+            return VX_OK;
+        }
+        limit = d->pf_rows - VX_PF_GRAIN;
     }
-    if (e != VX_OK) pf_free(d);
+    vx_error e = VX_OK;
+    for (int rows = R; rows > 0; rows -= VX_PF_GRAIN) {
+        pf_free(d);
+        if ((e = pf_alloc_rows(d, rows)) == VX_OK) {
+            d->pf_limit = limit;
+            return VX_OK;
+        }
+        limit = rows - VX_PF_GRAIN;
+    }
+    pf_free(d);
     return e;
 }
 
@@ -1290,11 +1308,13 @@ vx_error vx_dev_run_tokens(vx_model *m, const int *tokens, int n, int logits_mod
         /* long prompts: chunks of up to VX_PF_ROWS rows as one large-M batch */
         if (logits_mode != VX_LOGITS_ALL && pf_ok(d) && n - i >= d->opt.prefill_min_rows && c < n_ctx) {
             int P = n - i;
-            if (P > VX_PF_ROWS) P = VX_PF_ROWS;
+            if (P > pf_most(d)) P = pf_most(d);
             if (P > n_ctx - c) P = n_ctx - c;
             if (P >= d->opt.prefill_min_rows) {
                 if ((e = pf_alloc(d, P)) != VX_OK) return e;
                 if (P > d->pf_rows) P = d->pf_rows;
+            }
+            if (P >= d->opt.prefill_min_rows) {
                 const int last = i + P == n && logits_mode == VX_LOGITS_LAST;
                 if ((e = forward_prefill(m, tokens + i, P, c, last)) != VX_OK) return e;
                 if (last) TRY(vxh_download(logits_host, d->logits, sizeof(float) * (size_t)V, d->stream));

@@ -116,6 +116,7 @@ typedef struct vx_dev {
      * each [pf_rows][...] fp32, and the attention workspace for that many
      * rows */
     int pf_rows;                       /* rows the buffers hold (0: not allocated) */
+    int pf_limit;                      /* most rows there is room for (0: not found yet) */
     int pf_ws_ctx, pf_ws_cap;          /* n_ctx_alloc and attn_cap pf_ws was sized for */
     int *pf_tok;
     float *pf_x, *pf_qkv, *pf_q, *pf_att, *pf_gu;
