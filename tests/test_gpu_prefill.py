@@ -245,7 +245,8 @@ def test_rows_gemm_row_scales(P, typ, mag):
     assert ok, max_violation(g, o)
 
 
-@pytest.mark.parametrize("M,K", [(1, 32), (7, 1056), (64, 4096), (65, 96), (100, 11264), (9, 11296), (33, 22560),
+@pytest.mark.parametrize("M,K", [(1, 32), (7, 1056), (64, 4096), (65, 96), (5, 4128), (7, 8192), (7, 8224), (513, 8224),
+                                 (100, 11264), (9, 11296), (7, 12288), (7, 12320), (17, 18944), (33, 22560), (5, 24608),
                                  (1024, 96), (1030, 4096), (1025, 4128), (1024, 11296)])
 @pytest.mark.parametrize("kind", ["rmsnorm", "rmsnorm_w", "swiglu"])
 def test_rows_panel_kinds(P, kind, M, K):

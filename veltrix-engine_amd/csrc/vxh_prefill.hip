@@ -332,8 +332,15 @@ static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
 // workgroup per row the rows of a line go to 8 XCDs, whose L2s each write back
 // a part of it (2048 x 4096: 33 -> 19 us; norm and panel 50 -> 21; SwiGLU and
 // panel of 2048 x 11008 155 -> 62).  Few rows: a workgroup each (77 x 11008
-// 7.4 us, 22 with 8 rows: only 16 workgroups).  A row stays in registers, up
-// to KEEP groups of 8 columns per lane; what is left is read again.
+// 7.4 us, 22 with 8 rows: only 16 workgroups), of 4 wavefronts up to their
+// register window of 12288 columns, of 16 beyond (SwiGLU of 17 x 18944 21.0 ->
+// 12.1 us, 512 x 18944 50 -> 42), and SwiGLU rows of 16 from 8192 columns on
+// while a CU gets two of them or fewer (17 x 11008 10.8 -> 8.8 us, 512 x 11008
+// 28.4 -> 26.4; 1000 x 12288 52.6 against 55.9).  A row stays in registers, up
+// to KEEP groups of 8 columns per lane (2 up to 4096 columns, as groups past
+// the row's end cost their loads: norm of 1000 x 1024 8.4 -> 6.6 us); what is
+// left is read again (the sum of squares and the maximum come first), SwiGLU
+// evaluated again.
 enum { PF_ROWS = 0, PF_RMS = 1, PF_SWIGLU = 2 };
 
 template <int SRC, int KEEP, int PR, int WPR>
@@ -487,8 +494,13 @@ static int vx_pf_panel(const float *x, int ldx, int M, int K, const float *w, fl
     const int n_pairs = (K + 63) / 64;
     const unsigned rows = (unsigned)((M + PF_BM - 1) / PF_BM * PF_BM);
     float *rs = (float *)((char *)px + vx_pf_stage_bytes(M, K));
-    if (M < PF_MANY_ROWS)
+    const bool wide = K > 12 * 1024 || (SRC == PF_SWIGLU && K > 8 * 1024 && rows <= 512);
+    if (M < PF_MANY_ROWS && K <= 4 * 1024)
+        vx_pf_panel_kernel<SRC, 2, 1, 4><<<rows, 256, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px, rs);
+    else if (M < PF_MANY_ROWS && !wide)
         vx_pf_panel_kernel<SRC, 6, 1, 4><<<rows, 256, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px, rs);
+    else if (M < PF_MANY_ROWS)
+        vx_pf_panel_kernel<SRC, 3, 1, 16><<<rows, 1024, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px, rs);
     else if (K <= 4 * 1024)
         vx_pf_panel_kernel<SRC, 4, 8, 2><<<rows / 8, 1024, 0, vxh_hs(s)>>>(x, ldx, M, K, n_pairs, w, thr, (uint4 *)px,
                                                                          rs);
