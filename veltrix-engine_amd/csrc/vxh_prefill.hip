@@ -29,7 +29,7 @@ typedef uint32_t vx_u32x4 __attribute__((ext_vector_type(4)));
 struct vx_pf_args {
     const uint4 *wq;
     const uint32_t *wd;
-    int n_tiles, n_pairs, K;
+    int n_tiles, n_pairs;
     const uint4 *px;   // rows panel (vxh_rows_panel): [row group][pair][PF_STAGE units]
     const float *rs;   // [M] power-of-two row scales of the panel
     int M;
@@ -213,25 +213,41 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
 
 #pragma unroll
     for (int r = 0; r < 16; r += 4) add4(acc[NT - 1][MT - 1], r);
+    // Output (nt, mt, r) of a lane.  Loads of a batch are issued before its first
+    // store: behind a store that may alias them, every row scale would be a
+    // round trip of its own
     const int m0 = rg * PF_BM;
-    auto put = [&](int nt, int mt, int r, float sum) {
-        const int n = (T0 + nt) * 32 + c;
-        const int row = m0 + mt * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+    auto row_of = [&](int mt, int r) { return m0 + mt * 32 + 8 * (r / 4) + 4 * h + (r % 4); };
+    auto col_of = [&](int nt) { return (T0 + nt) * 32 + c; };
+    auto scale_of = [&](int mt, int r) { return a.rs[min(row_of(mt, r), a.M - 1)]; };
+    auto resid = [&](int nt, int mt, int r) {
+        return a.r[(size_t)min(row_of(mt, r), a.M - 1) * a.ldr + min(col_of(nt), a.n_out - 1)];
+    };
+    auto put = [&](int nt, int mt, int r, float sum, float rsv, float rv) {
+        const int n = col_of(nt), row = row_of(mt, r);
         if (n >= a.n_out || row >= a.M) return;
-        float v = (sum * a.rs[row]) * a.scale;   // the row scale is a power of two
-        if (a.r) v = a.r[(size_t)row * a.ldr + n] + v;
-        a.y[(size_t)row * a.ldy + n] = v;
+        const float v = (sum * rsv) * a.scale;   // the row scale is a power of two
+        a.y[(size_t)row * a.ldy + n] = a.r ? rv + v : v;
     };
     if constexpr (KS == 1) {
+        float rsv[MT][16];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) rsv[mt][r] = scale_of(mt, r);
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < MT; mt++) {
+                float rv[16];
 #pragma unroll
-                for (int r = 0; r < 16; r++) put(nt, mt, r, acc[nt][mt][r]);
+                for (int r = 0; r < 16; r++) rv[r] = a.r ? resid(nt, mt, r) : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) put(nt, mt, r, acc[nt][mt][r], rsv[mt][r], rv[r]);
+            }
     } else {
         // [ks][cw][register][lane]; the last step's barrier freed the stages
-        constexpr int R = NT * MT * 16;
+        constexpr int R = NT * MT * 16, RK = R / KS;
         static_assert(R % KS == 0, "registers of a tile over the K slices");
         float *red = (float *)lds;
 #pragma unroll
@@ -241,13 +257,20 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
 #pragma unroll
                 for (int r = 0; r < 16; r++) red[(wave * R + (nt * MT + mt) * 16 + r) * 64 + lane] = acc[nt][mt][r];
         __syncthreads();
+        float rsv[RK], rv[RK];
 #pragma unroll
-        for (int j = 0; j < R / KS; j++) {
-            const int reg = ks * (R / KS) + j;
+        for (int j = 0; j < RK; j++) {
+            const int reg = ks * RK + j;
+            rsv[j] = scale_of((reg / 16) % MT, reg % 16);
+            rv[j] = a.r ? resid(reg / (16 * MT), (reg / 16) % MT, reg % 16) : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < RK; j++) {
+            const int reg = ks * RK + j;
             float v = 0.0f;
 #pragma unroll
             for (int k = 0; k < KS; k++) v += red[((k * CW + cw) * R + reg) * 64 + lane];
-            put(reg / (16 * MT), (reg / 16) % MT, reg % 16, v);
+            put(reg / (16 * MT), (reg / 16) % MT, reg % 16, v, rsv[j], rv[j]);
         }
     }
 }
@@ -288,7 +311,7 @@ static int vx_pf_gemm_launch(const vx_pf_args &a, hipStream_t s)
 
 // Which split: the estimated time in rounds of workgroups over the 256 CUs.
 // Each weight is the measured time of one round, in units of 40 us at
-// K = 4096 (all splits scale with K alike):
+// K = 4096 (from there all splits scale with K alike):
 //   64 x 256, K whole: two workgroups to a CU; a full round of 512 takes 4.05,
 //     a last one of up to 256 (one to a CU) 2.  The best rate per tile, but
 //     M = 512, N = 4096 would leave half the CUs empty.
@@ -305,8 +328,15 @@ static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
     auto groups = [&](int tiles) { return n_rg * ((a.n_tiles + tiles - 1) / tiles); };
     auto rounds = [&](long n) { return (float)((n + 255) / 256); };
     const long n0 = groups(8), rest = n0 % 512;
-    const float t0 = 4.05f * (float)(n0 / 512) + (rest == 0 ? 0.0f : rest <= 256 ? 2.0f : 4.05f);
-    const float t1 = 1.1f * rounds(groups(4)), t2 = 0.65f * rounds(groups(2)), t3 = 0.38f * rounds(groups(1));
+    // a round's part that does not shrink with K (output rows, join of the K
+    // slices) from K = 64: 256 x 11008 x 128 by 64 x 128 12.8 us, by 64 x 64 15.9;
+    // 512 x 11008 x 64 with K whole 15.8, by 64 x 128 18.7
+    const float k = fminf((float)a.n_pairs / 64.0f, 1.0f);
+    auto weight = [&](float at4096, float fixed) { return k < 1.0f ? fixed + (at4096 - fixed) * k : at4096; };
+    const float full = weight(4.05f, 0.33f), half = weight(2.0f, 0.33f);
+    const float t0 = full * (float)(n0 / 512) + (rest == 0 ? 0.0f : rest <= 256 ? half : full);
+    const float t1 = weight(1.1f, 0.13f) * rounds(groups(4)), t2 = weight(0.65f, 0.12f) * rounds(groups(2)),
+                t3 = weight(0.38f, 0.06f) * rounds(groups(1));
     const float best = fminf(fminf(t0, t1), fminf(t2, t3));
     if (t0 == best) return vx_pf_gemm_launch<QT, 2, 4, 1>(a, s);
     if (t1 == best) return vx_pf_gemm_launch<QT, 2, 2, 4>(a, s);
@@ -547,7 +577,6 @@ extern "C" int vxh_gemm_rows(const vxh_qmat *W, const void *px, int M, float *Y,
     a.wd = (const uint32_t *)W->d;
     a.n_tiles = W->n_rows / 32;
     a.n_pairs = W->n_pairs;
-    a.K = W->n_cols;
     a.px = (const uint4 *)px;
     a.rs = (const float *)((const char *)px + vx_pf_stage_bytes(M, W->n_cols));
     a.M = M;
