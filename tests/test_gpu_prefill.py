@@ -1,6 +1,6 @@
 """Large-M prompt prefill (vx_model_forward of a long prompt: chunks of up to
-512 rows through vxh_gemm_rows, vxh_rope_kv_rows, vxh_attention and
-vxh_swiglu_rows) against the oracle, which runs the prompt one token per
+2048 rows through vxh_rmsnorm_rows_panel, vxh_gemm_rows, vxh_rope_kv_rows,
+vxh_attention_rows and vxh_swiglu_rows_panel) against the oracle, which runs the prompt one token per
 forward like the reference (src/speculative.c:100-107, src/model.c:391-628).
 
 Checked at the fp32 bar (1e-4 + 1e-3 |ref|): the last token's logits, every
@@ -140,8 +140,9 @@ def test_prefill_buffers_grow(P, tmp_path, d, h, kv):
         P.vx_model_destroy(mb)
 
 
-def _rows_gemm(P, typ, W, X, R=None, scale=1.0):
-    """vxh_rows_panel + vxh_gemm_rows on host arrays: Y = R + scale X W^T."""
+def _rows_gemm(P, typ, W, X, R=None, scale=1.0, in_place=False):
+    """vxh_rows_panel + vxh_gemm_rows on host arrays: Y = R + scale X W^T
+    (in_place: Y is R's buffer)."""
     vp = C.c_void_p
     L = N.bind_vxh(P)
     L.vxh_qmat_alloc.argtypes = [vp, C.c_int, C.c_int, C.c_int]
@@ -160,6 +161,9 @@ def _rows_gemm(P, typ, W, X, R=None, scale=1.0):
     px = N.DevBuf(L, nbytes=L.vxh_rows_panel_bytes(M, cols))
     dy = N.DevBuf(L, nbytes=4 * M * rows)
     dr = N.DevBuf(L, R) if R is not None else None
+    if in_place:
+        dy.free()
+        dy = dr
     try:
         assert L.vxh_rows_panel(dx.ptr, cols, M, cols, px.ptr, None) == 0, L.vxh_last_error()
         assert L.vxh_gemm_rows(C.byref(q), px.ptr, M, dy.ptr, rows, rows, dr.ptr if dr else None, rows, scale,
@@ -306,23 +310,49 @@ def test_rows_panel_kinds(P, kind, M, K):
         buf.free()
 
 
+SPLITS = ["64x256", "64x128 K/4", "64x64 K/8", "64x32 K/8"]
+
+
+def _rows_split(M, rows, cols):
+    """The split the dispatch takes, by its rule (rounds of workgroups times
+    the weight of one, of which a fixed part does not shrink with K)."""
+    f = np.float32
+    groups = lambda tiles: (M + 63) // 64 * (((rows + 31) // 32 + tiles - 1) // tiles)
+    k = f(min((cols + 63) // 64 / 64, 1.0))
+    weight = lambda w, fixed: f(w) if k == 1 else f(fixed) + (f(w) - f(fixed)) * k
+    n0 = groups(8)
+    last = f(0) if n0 % 512 == 0 else weight(2.0, 0.33) if n0 % 512 <= 256 else weight(4.05, 0.33)
+    t = [weight(4.05, 0.33) * f(n0 // 512) + last]
+    t += [weight(w, c) * f((groups(n) + 255) // 256) for w, c, n in ((1.1, 0.13, 4), (0.65, 0.12, 2), (0.38, 0.06, 1))]
+    return SPLITS[int(np.argmin(t))]
+
+
 @pytest.mark.parametrize("typ", [GGML_Q4_0, GGML_Q8_0])
-@pytest.mark.parametrize("M,rows,cols", [
-    (1, 1, 32), (17, 300, 128), (32, 96, 544), (33, 33, 1120), (65, 4096, 96), (96, 2080, 544),
-    (129, 21984, 64), (161, 11233, 160), (500, 4064, 288), (512, 4096, 96), (1025, 8224, 32), (2048, 4097, 96)])
-def test_rows_gemm_splits(P, typ, M, rows, cols):
+@pytest.mark.parametrize("M,rows,cols,split", [
+    (1, 1, 32, "64x32 K/8"), (17, 300, 128, "64x32 K/8"), (32, 96, 544, "64x32 K/8"), (33, 33, 1120, "64x32 K/8"),
+    (65, 4096, 96, "64x32 K/8"), (96, 2080, 544, "64x32 K/8"), (300, 8160, 4128, "64x32 K/8"),
+    (250, 4064, 288, "64x64 K/8"), (256, 4096, 64, "64x64 K/8"), (230, 4001, 4128, "64x64 K/8"),
+    (161, 11233, 160, "64x128 K/4"), (500, 4064, 288, "64x128 K/4"), (512, 4096, 96, "64x128 K/4"),
+    (1025, 8224, 32, "64x128 K/4"), (2048, 4097, 96, "64x128 K/4"), (500, 2049, 1056, "64x128 K/4"),
+    (129, 21984, 64, "64x256"), (600, 11233, 160, "64x256"), (540, 22001, 32, "64x256"), (512, 22016, 96, "64x256"),
+    (2048, 4096, 1056, "64x256"), (2048, 4096, 4128, "64x256")])
+def test_rows_gemm_splits(P, typ, M, rows, cols, split):
     """Every split of the prompt GEMM (64 x 32 and 64 x 64 with K over 8
-    wavefronts, 64 x 128 with K over 4, 64 x 256 with K whole) at ragged rows,
-    columns and K (one block, odd block counts, fewer pairs than K slices).
-    Bound per output: two fp16 parts keep each activation to 2^-22 of its
-    row's largest, and the fp32 sums round once per 16 products and twice per
-    block (the last term: at most 2^-24 of the sum of magnitudes each)."""
+    wavefronts, 64 x 128 with K over 4, 64 x 256 with K whole) at ragged rows
+    (last row groups of 1, 24 and up to 64 rows), columns and K (one block, odd
+    block counts, fewer pairs than K slices), the residual from a buffer of
+    its own and in place.  Bound per output: two fp16 parts keep each
+    activation to 2^-22 of its row's largest, and the fp32 sums round once per
+    16 products and twice per block (the last term: at most 2^-24 of the sum
+    of magnitudes each)."""
+    assert _rows_split(M, rows, cols) == split
     print(f"rows gemm split {'Q4_0' if typ == GGML_Q4_0 else 'Q8_0'} {M}x{rows}x{cols}", flush=True)
     rng = np.random.default_rng(M + rows + cols + typ)
     W = N.rand_q4_0(rng, rows, cols) if typ == GGML_Q4_0 else N.rand_q8_0(rng, rows, cols)
     X = rng.normal(0, 1, (M, cols)).astype(np.float32)
     R = rng.normal(0, 1, (M, rows)).astype(np.float32)
     Y = _rows_gemm(P, typ, W, X, R)
+    assert np.array_equal(Y, _rows_gemm(P, typ, W, X, R, in_place=True))
     w = N.q4_values(W) if typ == GGML_Q4_0 else N.q8_values(W)
     w = np.asarray(w, np.float64).reshape(rows, cols)
     prod, mag = X.astype(np.float64) @ w.T, np.abs(X).astype(np.float64) @ np.abs(w).T
