@@ -321,9 +321,9 @@ def _rows_split(M, rows, cols):
     k = f(min((cols + 63) // 64 / 64, 1.0))
     weight = lambda w, fixed: f(w) if k == 1 else f(fixed) + (f(w) - f(fixed)) * k
     n0 = groups(8)
-    last = f(0) if n0 % 512 == 0 else weight(2.0, 0.33) if n0 % 512 <= 256 else weight(4.05, 0.33)
-    t = [weight(4.05, 0.33) * f(n0 // 512) + last]
-    t += [weight(w, c) * f((groups(n) + 255) // 256) for w, c, n in ((1.1, 0.13, 4), (0.65, 0.12, 2), (0.38, 0.06, 1))]
+    last = f(0) if n0 % 512 == 0 else weight(2.0, 0.29) if n0 % 512 <= 256 else weight(4.05, 0.2)
+    t = [weight(4.05, 0.2) * f(n0 // 512) + last]
+    t += [weight(w, c) * f((groups(n) + 255) // 256) for w, c, n in ((1.1, 0.15, 4), (0.65, 0.1, 2), (0.38, 0.07, 1))]
     return SPLITS[int(np.argmin(t))]
 
 
@@ -332,9 +332,10 @@ def _rows_split(M, rows, cols):
     (1, 1, 32, "64x32 K/8"), (17, 300, 128, "64x32 K/8"), (32, 96, 544, "64x32 K/8"), (33, 33, 1120, "64x32 K/8"),
     (65, 4096, 96, "64x32 K/8"), (96, 2080, 544, "64x32 K/8"), (300, 8160, 4128, "64x32 K/8"),
     (250, 4064, 288, "64x64 K/8"), (256, 4096, 64, "64x64 K/8"), (230, 4001, 4128, "64x64 K/8"),
-    (161, 11233, 160, "64x128 K/4"), (500, 4064, 288, "64x128 K/4"), (512, 4096, 96, "64x128 K/4"),
-    (1025, 8224, 32, "64x128 K/4"), (2048, 4097, 96, "64x128 K/4"), (500, 2049, 1056, "64x128 K/4"),
-    (129, 21984, 64, "64x256"), (600, 11233, 160, "64x256"), (540, 22001, 32, "64x256"), (512, 22016, 96, "64x256"),
+    (130, 9000, 544, "64x128 K/4"), (200, 6001, 288, "64x128 K/4"), (500, 4064, 288, "64x128 K/4"),
+    (512, 4096, 96, "64x128 K/4"), (90, 11233, 1120, "64x128 K/4"), (500, 2049, 1056, "64x128 K/4"),
+    (161, 11233, 160, "64x256"), (1025, 8224, 32, "64x256"), (2048, 4097, 96, "64x256"), (129, 21984, 64, "64x256"),
+    (600, 11233, 160, "64x256"), (540, 22001, 32, "64x256"), (512, 22016, 96, "64x256"),
     (2048, 4096, 1056, "64x256"), (2048, 4096, 4128, "64x256")])
 def test_rows_gemm_splits(P, typ, M, rows, cols, split):
     """Every split of the prompt GEMM (64 x 32 and 64 x 64 with K over 8

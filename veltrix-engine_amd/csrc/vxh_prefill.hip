@@ -56,7 +56,7 @@ struct vx_pf_args {
 // LDS reads took as long as the products); the block sums of one tile are
 // scaled and added between the MFMAs of the next, so neither pipe waits.
 template <int QT, int NT, int CW, int KS, int MT>
-__device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int cg, vx_u32x4 *lds)
+__device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int cg, vx_u32x4 *lds, float *s_rs)
 {
     constexpr int WPP = QT == 2 ? 1 : 2;
     constexpr int RING = QT == 2 && CW != 2 ? 3 : 2;   // weight pairs in flight (register room)
@@ -116,6 +116,9 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
                     xf[blk][mt][s][hl] = __builtin_bit_cast(vx_half8, xp[(((mt * 2 + blk) * 2 + s) * 2 + hl) * 64]);
     };
 
+    // K whole: the row scales to LDS, for the epilogue (behind the first barrier)
+    const int m0 = rg * PF_BM;
+    if (KS == 1 && threadIdx.x < PF_BM) s_rs[threadIdx.x] = a.rs[min(m0 + (int)threadIdx.x, a.M - 1)];
     vx_f32x16 acc[NT][MT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
@@ -213,28 +216,22 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
 
 #pragma unroll
     for (int r = 0; r < 16; r += 4) add4(acc[NT - 1][MT - 1], r);
-    // Output (nt, mt, r) of a lane.  Loads of a batch are issued before its first
-    // store: behind a store that may alias them, every row scale would be a
-    // round trip of its own
-    const int m0 = rg * PF_BM;
-    auto row_of = [&](int mt, int r) { return m0 + mt * 32 + 8 * (r / 4) + 4 * h + (r % 4); };
+    // Output (nt, mt, r) of a lane.  Row scales (with K whole from LDS) and
+    // residual elements of a batch are read before its first store: behind a
+    // store that may alias them each would be a round trip of its own (2048 x
+    // 4096 x 4096 with the residual 161 -> 138 us, 2048 x 22016 x 128 80 -> 67)
+    auto row_of = [&](int mt, int r) { return mt * 32 + 8 * (r / 4) + 4 * h + (r % 4); };
     auto col_of = [&](int nt) { return (T0 + nt) * 32 + c; };
-    auto scale_of = [&](int mt, int r) { return a.rs[min(row_of(mt, r), a.M - 1)]; };
     auto resid = [&](int nt, int mt, int r) {
-        return a.r[(size_t)min(row_of(mt, r), a.M - 1) * a.ldr + min(col_of(nt), a.n_out - 1)];
+        return a.r[(size_t)min(m0 + row_of(mt, r), a.M - 1) * a.ldr + min(col_of(nt), a.n_out - 1)];
     };
     auto put = [&](int nt, int mt, int r, float sum, float rsv, float rv) {
-        const int n = col_of(nt), row = row_of(mt, r);
+        const int n = col_of(nt), row = m0 + row_of(mt, r);
         if (n >= a.n_out || row >= a.M) return;
-        const float v = (sum * rsv) * a.scale;   // the row scale is a power of two
+        const float v = (sum * (KS == 1 ? s_rs[row_of(mt, r)] : rsv)) * a.scale;   // the row scale is a power of two
         a.y[(size_t)row * a.ldy + n] = a.r ? rv + v : v;
     };
     if constexpr (KS == 1) {
-        float rsv[MT][16];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) rsv[mt][r] = scale_of(mt, r);
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
 #pragma unroll
@@ -243,7 +240,7 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
 #pragma unroll
                 for (int r = 0; r < 16; r++) rv[r] = a.r ? resid(nt, mt, r) : 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; r++) put(nt, mt, r, acc[nt][mt][r], rsv[mt][r], rv[r]);
+                for (int r = 0; r < 16; r++) put(nt, mt, r, acc[nt][mt][r], 0.0f, rv[r]);
             }
     } else {
         // [ks][cw][register][lane]; the last step's barrier freed the stages
@@ -261,7 +258,7 @@ __device__ __forceinline__ void vx_pf_gemm_body(const vx_pf_args &a, int rg, int
 #pragma unroll
         for (int j = 0; j < RK; j++) {
             const int reg = ks * RK + j;
-            rsv[j] = scale_of((reg / 16) % MT, reg % 16);
+            rsv[j] = a.rs[min(m0 + row_of((reg / 16) % MT, reg % 16), a.M - 1)];
             rv[j] = a.r ? resid(reg / (16 * MT), (reg / 16) % MT, reg % 16) : 0.0f;
         }
 #pragma unroll
@@ -287,6 +284,7 @@ template <int QT, int NT, int CW, int KS>
 __global__ __launch_bounds__(64 * CW *KS, 2) void vx_pf_gemm_kernel(vx_pf_args a, int n_cg, int n_rg)
 {
     __shared__ vx_u32x4 lds[vx_pf_lds_units<NT, CW, KS>()];
+    __shared__ float s_rs[KS == 1 ? PF_BM : 1];
     // workgroup id -> tile: ids go round the 8 XCDs, so every XCD takes a
     // contiguous run of tiles, in blocks of 8 row groups: the row groups of a
     // block share weight tiles and the columns share activation stages in L2
@@ -295,9 +293,9 @@ __global__ __launch_bounds__(64 * CW *KS, 2) void vx_pf_gemm_kernel(vx_pf_args a
     const int sup = id / (8 * n_cg), rs = min(8, n_rg - 8 * sup), in = id - sup * 8 * n_cg;
     const int rg = 8 * sup + in % rs, cg = in / rs;
     if (a.M - rg * PF_BM > 32)
-        vx_pf_gemm_body<QT, NT, CW, KS, 2>(a, rg, cg, lds);
+        vx_pf_gemm_body<QT, NT, CW, KS, 2>(a, rg, cg, lds, s_rs);
     else
-        vx_pf_gemm_body<QT, NT, CW, KS, 1>(a, rg, cg, lds);
+        vx_pf_gemm_body<QT, NT, CW, KS, 1>(a, rg, cg, lds, s_rs);
 }
 
 template <int QT, int NT, int CW, int KS>
@@ -328,15 +326,17 @@ static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
     auto groups = [&](int tiles) { return n_rg * ((a.n_tiles + tiles - 1) / tiles); };
     auto rounds = [&](long n) { return (float)((n + 255) / 256); };
     const long n0 = groups(8), rest = n0 % 512;
-    // a round's part that does not shrink with K (output rows, join of the K
-    // slices) from K = 64: 256 x 11008 x 128 by 64 x 128 12.8 us, by 64 x 64 15.9;
-    // 512 x 11008 x 64 with K whole 15.8, by 64 x 128 18.7
+    // Below K = 4096 a round has a part that does not shrink with K (output
+    // rows, join of the K slices).  Fitted to 100 shapes of K = 32 to 2048: the
+    // split taken is within 11% of the best one at each.  512 x 11008 x 128 with
+    // K whole 15.0 us, by 64 x 128 (its split at 4096) 18.5; 700 x 6000 x 128
+    // with K whole 14.6, by 64 x 64 23.9.
     const float k = fminf((float)a.n_pairs / 64.0f, 1.0f);
     auto weight = [&](float at4096, float fixed) { return k < 1.0f ? fixed + (at4096 - fixed) * k : at4096; };
-    const float full = weight(4.05f, 0.33f), half = weight(2.0f, 0.33f);
+    const float full = weight(4.05f, 0.2f), half = weight(2.0f, 0.29f);
     const float t0 = full * (float)(n0 / 512) + (rest == 0 ? 0.0f : rest <= 256 ? half : full);
-    const float t1 = weight(1.1f, 0.13f) * rounds(groups(4)), t2 = weight(0.65f, 0.12f) * rounds(groups(2)),
-                t3 = weight(0.38f, 0.06f) * rounds(groups(1));
+    const float t1 = weight(1.1f, 0.15f) * rounds(groups(4)), t2 = weight(0.65f, 0.1f) * rounds(groups(2)),
+                t3 = weight(0.38f, 0.07f) * rounds(groups(1));
     const float best = fminf(fminf(t0, t1), fminf(t2, t3));
     if (t0 == best) return vx_pf_gemm_launch<QT, 2, 4, 1>(a, s);
     if (t1 == best) return vx_pf_gemm_launch<QT, 2, 2, 4>(a, s);
