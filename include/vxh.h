@@ -376,7 +376,9 @@ int vxh_rope_kv_rows(const float *qkv, int ld_qkv, int M, int n_past, int n_ctx,
                      const float *cos_tab, const float *sin_tab, int n_pos, float *q_out, int ldq,
                      float *k_cache_layer, float *v_cache_layer, vxh_stream s);
 /* h[m][i] = |silu(g)| < thr ? 0 : silu(g) * u for the tile-interleaved gate/up
- * rows gu[M][ld_gu] (gate at 32(i/16) + i%16, up 16 further; src/model.c:582-585). */
+ * rows gu[M][ld_gu] (gate at 32(i/16) + i%16, up 16 further; src/model.c:582-585).
+ * For callers that need the fp32 rows; the prompt forward takes
+ * vxh_swiglu_rows_panel. */
 int vxh_swiglu_rows(const float *gu, int ld_gu, int M, int F, float thr, float *h, int ldh, vxh_stream s);
 
 /* ---- attention block ---------------------------------------------------------
@@ -483,6 +485,8 @@ int vxh_add_rows(float *y, int ldy, const float *x, int ldx, int M, int n, vxh_s
 /* dst[m][i] = src[m][i] for i < n. */
 int vxh_copy_rows(float *dst, int ld_dst, const float *src, int ld_src, int M, int n,
                   vxh_stream s);
+/* RMSNorm rows in fp32 (src/tensor.c:128-142), for callers that need them; the
+ * forwards take vxh_rmsnorm_panel and vxh_rmsnorm_rows_panel. */
 int vxh_rmsnorm(const float *x, int ldx, int M, int K, const float *w, float *out, int ld_out,
                 vxh_stream s);
 int vxh_fill_rows(float *y, int ld, int M, int col0, int n, float value, vxh_stream s);

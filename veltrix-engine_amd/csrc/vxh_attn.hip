@@ -831,9 +831,10 @@ struct vx_att_cfg {
 // bytes of the cache and the wavefronts of one chunk each.  Walking several
 // derives the q vectors once for all of them, streams the next chunk's K behind
 // this one's V and leaves fewer partials, as long as enough wavefronts remain:
-// * head_dim 128: 4 once one-chunk wavefronts take more than a round (3072
-//   resident): 9 rows x 28/4 heads over 8192 positions 41.7 -> 29.2 us, over 4009
-//   22.9 -> 18.1; over 3009 (3024 wavefronts) 19.3 against 20.0.
+// * head_dim 128: 4 from 3500 wavefronts of one chunk, past the 3072 that are
+//   resident at once: 9 rows x 28/4 heads over 8192 positions (8192 wavefronts)
+//   41.7 -> 29.2 us, over 4009 (4016) 22.9 -> 18.1; over 3009 (3024) one chunk
+//   takes 19.3 us and four 20.0.
 // * head_dim 64 (16 KB less per wavefront, more of them resident): 2 from 1200
 //   (9 x 32/4 over 1009: 12.2 -> 11.8), 4 from 6000 (16 x 14/2 over 8016: 22.8 ->
 //   18.3); at 4128 both 2 and 4 leave 9 x 32/32 over 2057 where it was.
@@ -899,10 +900,11 @@ __global__ __launch_bounds__(ATT_THREADS) __attribute__((amdgpu_waves_per_eu(HD 
 //    32 u + 8 (r/4) + 4 h + r % 4 of query n.  A tile's sums start from zero
 //    and join the running ones with the softmax rescale in one fma, so no fp32
 //    chain is longer than a tile.
-// Bound by the fp32 matrix rate (157 TFLOP/s).  2048 rows x 32 heads of
-// 128 from an empty cache 2363 -> 458 us, 512 over 2048 positions 590 -> 193 us
-// (16-query wavefronts that each read their K and V from L2 and wrote a partial
-// per 32 positions); 500 rows x 32/4 heads of 64 over 2036 240 -> 115 us.
+// Bound by the fp32 matrix rate (157 TFLOP/s).  Whole calls, join included:
+// 2048 rows x 32 heads of 128 from an empty cache 2364 -> 422 us, 512 over 2048
+// positions 590 -> 175 us (16-query wavefronts that each read their K and V from
+// L2 and wrote a partial per 32 positions); 500 rows x 32/4 heads of 64 over 2036
+// 210 -> 91 us.
 #define AR_Q 128                 // query vectors per workgroup
 #define AR_T 32                  // positions per tile
 
@@ -1252,8 +1254,9 @@ extern "C" size_t vxh_attention_workspace_floats(int M, int n_ctx, int cap, int 
 // more CUs (48 rows x 32 heads of 128 over 148 positions: 15.0 us there, 16.6
 // here; 100 x 8 x 64 over 600: 13.5 and 14.9); from it the prompt kernel is as
 // fast or faster (20 x 32 x 128 over 2020: 42.5 and 40.0; 100 x 32 x 128 over
-// 1100: 86 and 48).  Batches that the q|k|v kernel also takes (at most
-// VX_ATT_MFMA_MAX_M rows) keep its order of sums at any size.
+// 1100: 85 and 42).  Batches of at most VX_ATT_MFMA_MAX_M rows stay on the chunk
+// kernel at any size: 16 rows of G heads per kv head fill 16 G of a workgroup's
+// 128 query places.
 #define VX_ROWS_MIN_SCORES 1e6
 
 // Context segments of the prompt kernel, in whole tiles (*seg_t of them each):

@@ -49,9 +49,10 @@ struct vx_pf_args {
 // buffered with one barrier per step; with CW = 1 no two wavefronts share a
 // stage and each loads its operands straight into registers.
 //
-// Bound by the matrix cores once the chip is full: 2048 x 22016 x 4096 Q4_0
-// 1742 -> 750 us (2 products: 0.98 PFLOP/s, 85% of what a large library fp16
-// product reaches here), 512 x 22016 x 4096 532 -> 241 us.  64 x 64 per
+// Bound by the matrix cores once the chip is full (launches of the GEMM alone,
+// back to back): 2048 x 22016 x 4096 Q4_0 1714 -> 670 us (2 products: 1.10
+// PFLOP/s, 95% of what a large library fp16 product reaches here), 512 x 22016 x
+// 4096 441 -> 191 us.  64 x 64 per
 // wavefront because an operand read from LDS then feeds two MFMAs (at 64 x 32
 // LDS reads took as long as the products); the block sums of one tile are
 // scaled and added between the MFMAs of the next, so neither pipe waits.
@@ -308,17 +309,21 @@ static int vx_pf_gemm_launch(const vx_pf_args &a, hipStream_t s)
 }
 
 // Which split: the estimated time in rounds of workgroups over the 256 CUs.
-// Each weight is the measured time of one round, in units of 40 us at
-// K = 4096 (from there all splits scale with K alike):
+// Each weight is the time of one round relative to the others' at K = 4096
+// (from there all splits scale with K alike), as measured with an epilogue that
+// loaded element by element; with today's they are 3.1 (a last round 2.0), 1.0,
+// 0.55 and 0.36.  Weights refitted to 323 measured points chose splits 0.1%
+// faster on average, so these stay.  us back to back, Q4_0, before the K splits
+// and now:
 //   64 x 256, K whole: two workgroups to a CU; a full round of 512 takes 4.05,
 //     a last one of up to 256 (one to a CU) 2.  The best rate per tile, but
 //     M = 512, N = 4096 would leave half the CUs empty.
-//   64 x 128, K over 4: 1.1 a round.  512 x 4096 x 4096 113 -> 52 us (88 with K
-//     whole); 2048 x 4096 x 4096 199 us, where K whole takes 175.
-//   64 x 64, K over 8: 0.65 a round.  512 x 2048 x 5632 148 -> 44 us (64 with
-//     64 x 128); 128 x 22016 x 4096 160 -> 71 us (85 with K whole).
-//   64 x 32, K over 8: 0.38 a round.  77 x 4096 x 11008 Q8_0 269 -> 44 us (64
-//     with 64 x 64); 48 x 4096 x 4096 103 -> 18.5 us.
+//   64 x 128, K over 4: 1.1 a round.  512 x 4096 x 4096 100 -> 42 (78 with K
+//     whole); 2048 x 4096 x 4096 160, where K whole takes 132.
+//   64 x 64, K over 8: 0.65 a round.  512 x 2048 x 5632 135 -> 32 (51 with
+//     64 x 128); 128 x 22016 x 4096 150 -> 62 (78 with K whole).
+//   64 x 32, K over 8: 0.38 a round.  77 x 4096 x 11008 Q8_0 260 -> 35 (55
+//     with 64 x 64); 48 x 4096 x 4096 90 -> 12.7.
 template <int QT>
 static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
 {
