@@ -366,7 +366,7 @@ static int vx_pf_gemm(const vx_pf_args &a, hipStream_t s)
 // rows: 8 and 2, as the 16-byte units of 8 rows are one 128-byte line; with a
 // workgroup per row the rows of a line go to 8 XCDs, whose L2s each write back
 // a part of it (2048 x 4096: 33 -> 19 us; norm and panel 50 -> 21; SwiGLU and
-// panel of 2048 x 11008 155 -> 62).  Few rows: a workgroup each (77 x 11008
+// panel of 2048 x 11008 153 -> 70).  Few rows: a workgroup each (77 x 11008
 // 7.4 us, 22 with 8 rows: only 16 workgroups), of 4 wavefronts up to their
 // register window of 12288 columns, of 16 beyond (SwiGLU of 17 x 18944 21.0 ->
 // 12.1 us, 512 x 18944 50 -> 42), and SwiGLU rows of 16 from 8192 columns on
